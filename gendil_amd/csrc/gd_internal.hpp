@@ -34,6 +34,25 @@ struct FieldDev {
   const T* tab[kMaxTerms][kMaxDim];  // nullptr = factor 1
 };
 
+// The separable coefficients of a 3D plan as rows of 1D samples, in the order
+// sigma, beta, bc, mu.  A term is the product of its rows, one per axis its
+// mask names (bit d), in axis order; its scale is in its first row, and a term
+// without a factor has one z row holding its value.  A row has q + 2 samples
+// per element along its axis.
+enum { kTermSigma = 0, kTermBeta = 1, kTermBc = 4, kTermMu = 5, kTermFields = 6 };
+constexpr int kRowConstant = 3;
+constexpr int kMaxRows = kTermFields * kMaxTerms * 3;
+
+template <typename T>
+struct FieldTerms {
+  int first[kTermFields + 1];  // rows of field f: [first[f], first[f + 1])
+  int rank[kTermFields];
+  int mask[kTermFields];       // 3 bits per term
+  int axis[kMaxRows];          // kRowConstant: every sample is the scale
+  T scale[kMaxRows];
+  const T* tab[kMaxRows];      // of a constant row: readable, without meaning
+};
+
 // 1D tables for one (basis, n, q) pair, laid out contiguously on the device:
 // B[q][n] values, Gq[q][q] collocated derivative, b0[n], b1[n] face traces,
 // w[q] weights, xq[q] points, Gb[q][n] basis derivative, d0[n], d1[n] basis
@@ -67,6 +86,7 @@ struct Params {
   // coefficients
   int beta_kind;            // gd_beta_kind
   const FieldDev<T>* beta;  // [dim] (separable)
+  const FieldTerms<T>* terms;  // 3D plans
   const FieldDev<T>* sigma;
   const FieldDev<T>* bc;
   int bc_mode;
@@ -149,6 +169,11 @@ struct gd_plan {
   std::vector<gd::FieldDev<double>> fields64_host;  // host copies of the device descriptors
   std::vector<gd::FieldDev<float>> fields32_host;
   std::vector<void*> field_tables;  // device table allocations
+  // 3D plans: the terms list behind the descriptors in fields64 / fields32
+  const gd::FieldTerms<double>* terms64 = nullptr;
+  const gd::FieldTerms<float>* terms32 = nullptr;
+  int term_first[gd::kTermFields + 1] = {};  // host copies of FieldTerms::first, rank, mask
+  int term_rank[gd::kTermFields] = {}, term_mask[gd::kTermFields] = {};
   // autotuned 3D kernel choice ([0] FP64, [1] FP32): -1 = not tuned,
   // 0 = generic kernel, 1/2/4 = register kernel with that many lanes per
   // element, 16 + lanes = Kronecker-factored kernel

@@ -248,6 +248,57 @@ void free_fields(gd_plan* p)
   p->fields64 = p->fields32 = nullptr;
 }
 
+// One allocation and one copy: the field descriptors and, for 3D plans, the
+// terms list built from them (fields f: [0..3) beta, 3 sigma, 4 bc, 5 mu).
+template <typename T>
+int upload_descriptors(gd_plan* p, const std::vector<FieldDev<T>>& f, void** dst, const FieldTerms<T>** terms)
+{
+  const size_t head = f.size() * sizeof(FieldDev<T>);
+  std::vector<char> blob(head + (p->dim == 3 ? sizeof(FieldTerms<T>) : 0));
+  std::memcpy(blob.data(), f.data(), head);
+  GD_HIP(hipMalloc(dst, blob.size()));
+  if (p->dim == 3) {
+    static const int from[kTermFields] = {3, 0, 1, 2, 4, 5};  // sigma, beta, bc, mu
+    FieldTerms<T> t;
+    std::memset(&t, 0, sizeof(t));
+    int n = 0;
+    for (int i = 0; i < kTermFields; ++i) {
+      const FieldDev<T>& src = f[from[i]];
+      t.first[i] = n;
+      t.rank[i] = src.rank;
+      for (int r = 0; r < src.rank; ++r) {
+        T scale = src.scale[r];
+        int bits = 0;
+        for (int d = 0; d < 3; ++d)
+          if (src.tab[r][d]) {
+            bits |= 1 << d;
+            t.axis[n] = d;
+            t.scale[n] = scale;
+            t.tab[n++] = src.tab[r][d];
+            scale = T(1);
+          }
+        if (!bits) {
+          bits = 4;
+          t.axis[n] = kRowConstant;
+          t.scale[n] = scale;
+          t.tab[n++] = static_cast<const T*>(*dst);  // this block: longer than the q + 2 samples of one element
+        }
+        t.mask[i] |= bits << (3 * r);
+      }
+    }
+    t.first[kTermFields] = n;
+    for (int i = 0; i <= kTermFields; ++i) p->term_first[i] = t.first[i];
+    for (int i = 0; i < kTermFields; ++i) {
+      p->term_rank[i] = t.rank[i];
+      p->term_mask[i] = t.mask[i];
+    }
+    std::memcpy(blob.data() + head, &t, sizeof(t));
+  }
+  GD_HIP(hipMemcpy(*dst, blob.data(), blob.size(), hipMemcpyHostToDevice));
+  *terms = p->dim == 3 ? reinterpret_cast<const FieldTerms<T>*>(static_cast<char*>(*dst) + head) : nullptr;
+  return GD_OK;
+}
+
 // Upload beta[0..dim), sigma, bc, diffusivity as FieldDev arrays (double and
 // float).
 int upload_fields(gd_plan* p)
@@ -287,10 +338,8 @@ int upload_fields(gd_plan* p)
   }
   p->fields64_host = f64;
   p->fields32_host = f32;
-  GD_HIP(hipMalloc(&p->fields64, nf * sizeof(FieldDev<double>)));
-  GD_HIP(hipMalloc(&p->fields32, nf * sizeof(FieldDev<float>)));
-  GD_HIP(hipMemcpy(p->fields64, f64.data(), nf * sizeof(FieldDev<double>), hipMemcpyHostToDevice));
-  GD_HIP(hipMemcpy(p->fields32, f32.data(), nf * sizeof(FieldDev<float>), hipMemcpyHostToDevice));
+  if (int rc = upload_descriptors(p, f64, &p->fields64, &p->terms64)) return rc;
+  if (int rc = upload_descriptors(p, f32, &p->fields32, &p->terms32)) return rc;
   return GD_OK;
 }
 
@@ -341,9 +390,11 @@ Params<T> make_params(const gd_plan* p, const TableSet* ts, T mass_coef, T adv_c
   if constexpr (std::is_same_v<T, double>) {
     k.tab = ts->t64;
     k.beta = static_cast<const FieldDev<double>*>(p->fields64);
+    k.terms = p->terms64;
   } else {
     k.tab = ts->t32;
     k.beta = static_cast<const FieldDev<float>*>(p->fields32);
+    k.terms = p->terms32;
   }
   k.sigma = k.beta + D;
   k.bc = (p->bc_mode == GD_BC_INFLOW && p->bc_host.rank > 0) ? k.beta + D + 1 : nullptr;

@@ -1,0 +1,99 @@
+"""The plane kernel (uniform 3D apply for any basis, rule and separable or
+affine field) against the CPU oracle.
+
+Sizes: one cell, one-cell axes (periodic: an element is its own neighbour), a
+mesh smaller than a block, meshes whose last block is partly filled.  Every
+compiled (nodes, points) pair, both bases, both precisions; fields over one,
+two and three coordinates, fields whose sign changes within a face, affine
+fields; no, zero and polynomial inflow data.  Tolerances as for every other
+kernel: 1e-12 (FP64) and 1e-5 (FP32) relative L2."""
+import numpy as np
+import pytest
+import torch
+
+import gendil_amd as G
+import oracle
+from cases import TWO_PI, bc_field, beta_field, rel_l2, sigma_field
+from gendil_amd.fields import SeparableField, VectorField
+
+pytestmark = pytest.mark.gpu
+
+PLANE = 72
+PAIRS = [(2, 2), (2, 3), (2, 4), (3, 3), (3, 4), (3, 5), (4, 4), (4, 5), (4, 6), (5, 5), (5, 6)]
+
+
+def field(kind):
+    if kind == "mixed":  # rank 2 and 3, one to three coordinates, both signs within a face
+        return VectorField([
+            SeparableField([(0.3, {}), (1.0, {1: lambda s: np.sin(TWO_PI * s), 2: lambda s: np.cos(TWO_PI * s)})]),
+            SeparableField([(-0.2, {0: lambda s: s}), (0.7, {0: lambda s: np.cos(TWO_PI * s), 1: lambda s: s,
+                                                             2: lambda s: 1.0 - s}), (0.1, {2: lambda s: s})]),
+            SeparableField([(1.0, {0: lambda s: 0.4 - s})]),
+        ])
+    if kind == "affine":
+        return G.AffineField(np.array([[0.3, -1.0, 0.2], [0.9, 0.1, -0.4], [-0.5, 0.6, 0.7]]), np.array([0.1, -0.2, 0.05]))
+    return beta_field(kind, 3)
+
+
+def space(sizes, p, basis, periodic):
+    h = [0.9 / s * (1.0 + 0.2 * d) for d, s in enumerate(sizes)]
+    mesh = G.CartesianMesh(sizes, h, [0.1, -0.2, 0.3], periodic)
+    fe = G.MakeLobattoFiniteElement(p) if basis == "L" else G.MakeLegendreFiniteElement(p)
+    return G.MakeFiniteElementSpace(mesh, fe)
+
+
+def check(fes, q, dtype, beta, bc, sigma, mc, ac):
+    ir = G.MakeIntegrationRule(q)
+    g = bc_field(bc, 3)
+    if ac == 0.0:
+        op = G.MakeMassFiniteElementOperator(fes, ir, sigma)
+        kw = {}
+    else:
+        op = G.MakeMassAdvectionOperator(fes, ir, beta, sigma=sigma, bc=g, mass_coef=mc, adv_coef=ac)
+        kw = dict(adv_coef=ac, adv=beta, bc=g)
+    op.plan.set_variant(dtype, PLANE)
+    assert op.plan.query_variant(dtype, mc, ac) == PLANE
+    x = G.fill_random(op.num_dofs, 11)
+    y = torch.full((op.num_dofs,), float("nan"), dtype=dtype, device="cuda")
+    op(torch.as_tensor(x, dtype=dtype, device="cuda"), y)
+    if mc != 0.0:
+        kw.update(mass_coef=mc, sigma=sigma)
+    xr = x.astype(np.float32).astype(np.float64) if dtype == torch.float32 else x
+    ref = oracle.Problem(fes, ir, **kw).apply(xr)
+    assert rel_l2(y.double().cpu().numpy(), ref) <= (1e-12 if dtype == torch.float64 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("basis", ["L", "G"])
+@pytest.mark.parametrize("n,q", PAIRS)
+def test_step_every_pair(n, q, basis, dtype):
+    fes = space((5, 3, 4), n - 1, basis, [True, False, True])
+    check(fes, q, dtype, field("mixed"), "poly", sigma_field("poly", 3), 0.7, 0.4)
+
+
+@pytest.mark.parametrize("sizes", [(1, 1, 1), (1, 5, 1), (7, 1, 2), (33, 1, 1), (13, 11, 17)], ids=str)
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("kind,bc", [("mixed", "none"), ("affine", "zero"), ("affine", "poly"), ("const", "poly")])
+def test_advection_sizes_and_boundaries(sizes, periodic, kind, bc):
+    check(space(sizes, 2, "L", periodic), 4, torch.float64, field(kind), bc, None, 0.0, 1.0)
+
+
+@pytest.mark.parametrize("n,q", [(2, 4), (3, 5), (4, 6), (5, 6)])
+@pytest.mark.parametrize("sizes", [(1, 1, 1), (9, 5, 3)], ids=str)
+def test_mass(n, q, sizes):
+    for dtype in (torch.float64, torch.float32):
+        check(space(sizes, n - 1, "G", False), q, dtype, None, "none", sigma_field("poly", 3), 1.0, 0.0)
+
+
+def test_default_where_no_faster_kernel_serves():
+    """The plane kernel is the default for rules, bases and fields that the Kronecker and register kernels refuse;
+    0 pins the generic kernel."""
+    fes = space((6, 5, 4), 3, "L", False)
+    op = G.MakeAdvectionOperator(fes, G.MakeIntegrationRule(5), field("mixed"))
+    assert op.plan.query_variant(torch.float64, 0.0, 1.0) == PLANE
+    op.plan.set_variant(torch.float64, 0)
+    assert op.plan.query_variant(torch.float64, 0.0, 1.0) == 0
+    x = torch.as_tensor(G.fill_random(op.num_dofs, 2), device="cuda")
+    generic = op(x, torch.empty_like(x)).cpu().numpy()
+    op.plan.set_variant(torch.float64, -1)
+    assert rel_l2(op(x, torch.empty_like(x)).cpu().numpy(), generic) <= 1e-13
