@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "gd_diff.hpp"
+#include "gd_dplane_api.hpp"
 
 namespace gd {
 namespace {
@@ -37,6 +38,10 @@ int diff_apply(const gd_plan* plan, const T* x, T* y, hipStream_t s)
   if (!ks)
     return fail(GD_ERR_UNSUPPORTED, "no diffusion kernel compiled for dim=" + std::to_string(plan->dim) +
                                         " nodes=" + std::to_string(N) + " quad=" + std::to_string(Q));
+  if (plan->dim == 3) {
+    const int rc = pl::apply_diffusion<T>(plan, x, y, s);
+    if (rc != GD_ERR_UNSUPPORTED) return rc;
+  }
   const TableSet* ts = find_tables(plan, N, Q);
   if (!ts) return fail(GD_ERR_INVALID, "plan has no tables for its own rule");
   const Params<T> prm = make_params<T>(plan, ts, T(0), T(0));

@@ -13,7 +13,7 @@ import torch
 
 import gendil_amd as G
 import oracle
-from cases import TWO_PI, bc_field, beta_field, rel_l2, sigma_field
+from cases import TWO_PI, bc_field, beta_field, diffusivity_field, rel_l2, sigma_field
 from gendil_amd.fields import SeparableField, VectorField
 
 pytestmark = pytest.mark.gpu
@@ -97,3 +97,33 @@ def test_default_where_no_faster_kernel_serves():
     generic = op(x, torch.empty_like(x)).cpu().numpy()
     op.plan.set_variant(torch.float64, -1)
     assert rel_l2(op(x, torch.empty_like(x)).cpu().numpy(), generic) <= 1e-13
+
+
+DIFF_PAIRS = [(2, 3), (2, 4), (3, 3), (3, 4), (3, 5), (4, 4), (4, 5), (4, 6)]
+
+
+def check_diffusion(fes, q, dtype, mu, sigma, kappa):
+    ir = G.MakeIntegrationRule(q)
+    op = G.MakeDiffusionOperator(fes, ir, mu, sigma, kappa)
+    x = G.fill_random(op.num_dofs, 13)
+    y = torch.full((op.num_dofs,), float("nan"), dtype=dtype, device="cuda")
+    op(torch.as_tensor(x, dtype=dtype, device="cuda"), y)
+    xr = x.astype(np.float32).astype(np.float64) if dtype == torch.float32 else x
+    ref = oracle.Problem(fes, ir).diffusion(xr, mu, sigma, kappa)
+    assert rel_l2(y.double().cpu().numpy(), ref) <= (1e-12 if dtype == torch.float64 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("basis", ["L", "G"])
+@pytest.mark.parametrize("n,q", DIFF_PAIRS)
+def test_diffusion_every_pair(n, q, basis, dtype):
+    """The diffusion plane kernel, an eight-term diffusivity, mixed boundaries."""
+    check_diffusion(space((5, 3, 4), n - 1, basis, [True, False, True]), q, dtype, diffusivity_field("trig", 3), -1.0, 9.0)
+
+
+@pytest.mark.parametrize("sizes", [(1, 1, 1), (1, 5, 1), (33, 1, 1), (13, 11, 7)], ids=str)
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("rank", [0, 1, 2, 3])
+def test_diffusion_sizes_ranks_and_boundaries(sizes, periodic, rank):
+    terms = [(1.5, {}), (0.3, {0: lambda s: s, 2: lambda s: 1.0 + s}), (0.2, {1: lambda s: s * s})][:rank]
+    check_diffusion(space(sizes, 3, "L", periodic), 5, torch.float64, SeparableField(terms), 1.0 if rank == 2 else 0.0, 4.0)
