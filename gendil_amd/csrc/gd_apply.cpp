@@ -10,6 +10,7 @@
 #include "gd_k3k_api.hpp"
 #include "gd_n2k_api.hpp"
 #include "gd_padapt_api.hpp"
+#include "gd_padj_api.hpp"
 #include "gd_plane_api.hpp"
 
 namespace gd {
@@ -218,6 +219,8 @@ int gd_apply_T_f64(const gd_plan* plan, double mass_coef, double adv_coef, const
   if (adv_coef == 0.0) return ks->fwd64_mass(prm, r, z, (hipStream_t)stream);  // M is symmetric
   rc = gd::check_adv(plan, false);
   if (rc) return rc;
+  rc = gd::pl::apply_transpose(plan, mass_coef, adv_coef, r, z, (hipStream_t)stream);
+  if (rc != GD_ERR_UNSUPPORTED) return rc;
   return ks->trn64(prm, r, z, (hipStream_t)stream);
 }
 
@@ -353,13 +356,14 @@ int gd_adv_grad_beta_f64(const gd_plan* plan, double adv_coef, const double* u, 
   rc = gd::check_adv(plan, true);
   if (rc) return rc;
   if (!u || !r || !dbeta_cell || !dbeta_face) return fail(GD_ERR_INVALID, "null argument");
+  for (int d = 0; d < plan->dim; ++d)
+    if (!dbeta_face[d]) return fail(GD_ERR_INVALID, "null face gradient array");
+  rc = gd::pl::grad_beta(plan, adv_coef, u, r, dbeta_cell, dbeta_face, (hipStream_t)stream);
+  if (rc != GD_ERR_UNSUPPORTED) return rc;
   const gd::TableSet* ts = gd::find_tables(plan, plan->desc.order + 1, plan->desc.num_quad);
   gd::Params<double> prm = gd::make_params<double>(plan, ts, 0.0, adv_coef);
   prm.dbeta_cell = dbeta_cell;
-  for (int d = 0; d < plan->dim; ++d) {
-    if (!dbeta_face[d]) return fail(GD_ERR_INVALID, "null face gradient array");
-    prm.dbeta_face[d] = dbeta_face[d];
-  }
+  for (int d = 0; d < plan->dim; ++d) prm.dbeta_face[d] = dbeta_face[d];
   // the kernel reads r through its second vector argument
   return ks->grad64(prm, u, const_cast<double*>(r), (hipStream_t)stream);
 }

@@ -80,16 +80,37 @@ struct Args {
   FastDiv d0, d1;
   int M[3];
   int periodic_mask;
-  int gll, affine;   // instance: traces are node layers; beta is affine
+  int gll, field;    // instance: traces are node layers; how beta is given
   int bc_none;       // boundary faces carry no flux
   int bc_data;       // inflow data with at least one term
   T h[3], invh[3], origin[3];
   T detJ, mass_coef, adv_coef;
   T affA[3][3], affc[3];
+  const T *beta_cell, *beta_face[3];  // pointwise beta
   const FieldTerms<T>* terms;
   const FieldDev<T>* sigma_tab;
   const T *B, *Gb, *b0, *b1, *xq, *w;
 };
+
+enum { kSeparable = 0, kAffine = 1, kPointwise = 2 };
+
+// number of element sub's lower (0) or upper (1) face normal to axis a, in the
+// order of the per-face-point arrays (extents M, along a M + 1 unless periodic)
+template <typename A>
+__device__ __forceinline__ int64_t face_index(const A& a, const int* sub, int ax, int side)
+{
+  const bool per = (a.periodic_mask >> ax) & 1;
+  int s[3] = {sub[0], sub[1], sub[2]};
+  int64_t ext[2] = {a.M[0], a.M[1]};
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (d == ax) {
+      s[d] += side;
+      if (per && s[d] == a.M[d]) s[d] = 0;
+      if (d < 2) ext[d] += per ? 0 : 1;
+    }
+  return s[0] + ext[0] * (s[1] + ext[1] * s[2]);
+}
 
 // scalar (constant address space) view of a table: uniform reads become
 // scalar loads whatever the surrounding stores
@@ -168,7 +189,7 @@ struct Geo {
   static constexpr int PL = ADV ? Q + 2 : Q;
   // most elements per block: two z faces each fill the last wave; the mass
   // planes fill two waves
-  static constexpr int EPB = 32;
+  static constexpr int EPB = N >= 5 ? 128 / Q : 32;
   static constexpr int CELLW = (EPB * Q + 63) / 64 * 64;  // waves that take cell planes in phase 2
   static constexpr int NT = ADV ? CELLW + 64 : (CELLW < 128 ? 128 : CELLW);
 };
@@ -344,6 +365,14 @@ struct Planes {
     }
   }
 
+  __device__ __forceinline__ static void plane_of(const T* src, T (&b)[Q][Q])
+  {
+#pragma unroll
+    for (int k = 0; k < Q; ++k)
+#pragma unroll
+      for (int j = 0; j < Q; ++j) b[k][j] = src[k * Q + j];
+  }
+
   // out[j] = sum_i tab[j][i] in[i]: n nodes to q points
   template <class Tab>
   __device__ __forceinline__ static void up(const Tab& tab, const T (&in)[N], T (&out)[Q])
@@ -412,8 +441,8 @@ struct Planes {
 };
 
 // GLL: the basis values at the element ends are unit vectors, so a trace is a
-// node layer.  AFF: beta is affine, else separable.
-template <typename T, int N, int Q, bool ADV, bool GLL, bool AFF>
+// node layer.  FIELD: how beta is given (kSeparable, kAffine, kPointwise).
+template <typename T, int N, int Q, bool ADV, bool GLL, int FIELD>
 __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
     plane_kernel(Args<T> a, const T* __restrict__ x, T* __restrict__ y)
 {
@@ -454,15 +483,32 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
   };
 
   auto rows = [](const T* sm) { return LdsRows<T, Q + 2>{sm}; };
-  // the advection field times the weights of its plane (times wz) or line
-  auto beta_at = [&](int c, const int* sub, const T* sm, int kz, T wz, T (&b)[Q][Q]) {
-    if constexpr (AFF) P::affine(a, c, sub, kz, w, wz, b);
-    else P::template separable<true>(a.beta[c], rows(sm), kz, w, wz, b);
+  // the advection field times the weights of its plane (times wz) or line; a
+  // pointwise field's plane comes without (its weights go into v)
+  auto beta_at = [&](int c, int e, const int* sub, const T* sm, int kz, T wz, T (&b)[Q][Q]) {
+    if constexpr (FIELD == kAffine) P::affine(a, c, sub, kz, w, wz, b);
+    else if constexpr (FIELD == kPointwise) {
+      const T* src = kz < Q ? a.beta_cell + ((int64_t)e * 3 + c) * (Q * Q * Q) + kz * (Q * Q)
+                            : a.beta_face[2] + face_index(a, sub, 2, kz - Q) * (Q * Q);
+      P::plane_of(src, b);
+    } else P::template separable<true>(a.beta[c], rows(sm), kz, w, wz, b);
   };
   auto beta_ends = [&](auto ax, const int* sub, const T* sm, int kz, T wz, T (&b)[2][Q]) {
     constexpr int AX = decltype(ax)::value;
-    if constexpr (AFF) P::template affine_ends<AX>(a, sub, kz, w, wz, b);
-    else P::template separable_ends<AX, true>(a.beta[AX], rows(sm), kz, w, wz, b);
+    if constexpr (FIELD == kAffine) P::template affine_ends<AX>(a, sub, kz, w, wz, b);
+    else if constexpr (FIELD == kPointwise) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const T* src = a.beta_face[AX] + face_index(a, sub, AX, s) * (Q * Q) + kz * Q;
+#pragma unroll
+        for (int k = 0; k < Q; ++k) b[s][k] = src[k];
+      }
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        b[0][k] *= wz * w[k];
+        b[1][k] *= wz * w[k];
+      }
+    } else P::template separable_ends<AX, true>(a.beta[AX], rows(sm), kz, w, wz, b);
   };
 
   // ---- phase 1: z contractions of the own and the neighbours' pencils ----
@@ -633,6 +679,12 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
           for (int i = 0; i < N; ++i) u[m][i] = r[m * N + i];
         P::template interp<GLL>(B, u, v, xo, b0, b1);
       }
+      if constexpr (ADV && FIELD == kPointwise) {
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+#pragma unroll
+          for (int j = 0; j < Q; ++j) v[k][j] *= wz * w[k] * w[j];
+      }
       T A[N][N];
 #pragma unroll
       for (int m = 0; m < N; ++m)
@@ -680,7 +732,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
               pin(fx[s]);
             }
           }
-          beta_at(0, sub, sm, kz, wz, b);
+          beta_at(0, e, sub, sm, kz, wz, b);
 #pragma unroll
           for (int k = 0; k < Q; ++k) {
             T f[Q], g[N];
@@ -744,7 +796,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
               }
             }
           }
-          beta_at(1, sub, sm, kz, wz, b);
+          beta_at(1, e, sub, sm, kz, wz, b);
 #pragma unroll
           for (int k = 0; k < Q; ++k) {
             T f[Q], g[N];
@@ -771,7 +823,8 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
         }
       } else if (a.mass_coef != T(0)) {
         const T c = a.mass_coef * a.detJ;
-        P::template separable<true>(a.sigma, rows(sm), kz, w, wz, b);
+        if constexpr (FIELD == kPointwise) P::template separable<false>(a.sigma, rows(sm), kz, w, T(1), b);
+        else P::template separable<true>(a.sigma, rows(sm), kz, w, wz, b);
 #pragma unroll
         for (int k = 0; k < Q; ++k) {
           T f[Q], g[N];
@@ -785,7 +838,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
       }
       if constexpr (ADV) {  // z component: tested with B' in z, kept apart
         const T c = a.adv_coef * a.detJ * a.invh[2];
-        beta_at(2, sub, sm, kz, wz, b);
+        beta_at(2, e, sub, sm, kz, wz, b);
         // the part tested with B in z leaves first: its registers are free
         // for this one.  The record's inputs are all consumed by here.
 #pragma unroll
@@ -825,7 +878,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
       T* r = rec + (el * PL + Q + s) * PITCH;
       const T* sm = smp + el * a.spitch;
       T b[Q][Q], u[N][N], A[N][N];
-      beta_at(2, sub, sm, Q + s, T(1), b);
+      beta_at(2, e, sub, sm, Q + s, T(1), b);
       const bool bnd = neighbour(e, sub, 2, s) < 0;
       const T c = bnd && a.bc_none ? T(0) : a.adv_coef * a.detJ * a.invh[2];
 #pragma unroll
@@ -845,6 +898,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
         for (int j = 0; j < Q; ++j) {
           const T dot = s ? b[k][j] : -b[k][j];
           f[j] = c * (dot > T(0) ? dot * own[j] : dot * ext[j]);
+          if constexpr (FIELD == kPointwise) f[j] *= w[k] * w[j];
         }
         P::down(B, f, g);
 #pragma unroll

@@ -21,12 +21,10 @@ const Entry* find(int N, int Q)
   return nullptr;
 }
 
-// 3D, uniform order, a field evaluated from tables or affine; element and
-// neighbour numbers in 32 bits
+// 3D, uniform order; element and neighbour numbers in 32 bits
 const Entry* serving(const gd_plan* plan, bool adv)
 {
   if (plan->dim != 3 || plan->padapt || plan->E >= (int64_t)1 << 31) return nullptr;
-  if (adv && plan->beta_kind != GD_BETA_SEPARABLE && plan->beta_kind != GD_BETA_AFFINE) return nullptr;
   return find(plan->desc.order + 1, plan->desc.num_quad);
 }
 
@@ -70,7 +68,11 @@ int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStr
   a.mass_coef = mass_coef;
   a.adv_coef = adv_coef;
   a.gll = plan->desc.basis == GD_BASIS_GLL;
-  a.affine = plan->beta_kind == GD_BETA_AFFINE;
+  a.field = plan->beta_kind == GD_BETA_AFFINE ? kAffine : (plan->beta_kind == GD_BETA_POINTWISE ? kPointwise : kSeparable);
+  if constexpr (std::is_same_v<T, double>) {
+    a.beta_cell = plan->beta_cell;
+    for (int d = 0; d < 3; ++d) a.beta_face[d] = plan->beta_face[d];
+  }
   a.bc_none = plan->bc_mode == GD_BC_NONE;
   a.bc_data = !a.bc_none && plan->bc_host.rank > 0;
   const Tables1D<T>* tab;

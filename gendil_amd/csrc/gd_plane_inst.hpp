@@ -8,7 +8,7 @@
 namespace gd {
 namespace pl {
 
-template <typename T, int N, int Q, bool ADV, bool GLL, bool AFF>
+template <typename T, int N, int Q, bool ADV, bool GLL, int FIELD>
 int launch_kind(Args<T>& a, const T* x, T* y, hipStream_t s)
 {
   using G = Geo<N, Q, ADV>;
@@ -20,7 +20,7 @@ int launch_kind(Args<T>& a, const T* x, T* y, hipStream_t s)
   while (a.epb > 4 && ((int64_t)a.epb * 512 > a.E || (size_t)a.epb * per > 80 * 1024)) a.epb = (a.epb + 1) / 2;
   a.num_blocks = (int)((a.E + a.epb - 1) / a.epb);
   const size_t lds = a.epb * per;
-  auto kern = plane_kernel<T, N, Q, ADV, GLL, AFF>;
+  auto kern = plane_kernel<T, N, Q, ADV, GLL, FIELD>;
   if (lds > 160 * 1024) return GD_ERR_UNSUPPORTED;
   if (lds > 64 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -35,12 +35,15 @@ int launch_kind(Args<T>& a, const T* x, T* y, hipStream_t s)
 template <typename T, int N, int Q, bool ADV>
 int launch(Args<T>& a, const T* x, T* y, hipStream_t s)
 {
-  if constexpr (!ADV) return launch_kind<T, N, Q, false, true, false>(a, x, y, s);  // no traces, no beta
+  if constexpr (!ADV) return launch_kind<T, N, Q, false, true, kSeparable>(a, x, y, s);  // no traces, no beta
   else {
-    if (a.gll) return a.affine ? launch_kind<T, N, Q, true, true, true>(a, x, y, s)
-                        : launch_kind<T, N, Q, true, true, false>(a, x, y, s);
-    return a.affine ? launch_kind<T, N, Q, true, false, true>(a, x, y, s)
-               : launch_kind<T, N, Q, true, false, false>(a, x, y, s);
+    if constexpr (sizeof(T) == 8)
+      if (a.field == kPointwise) return a.gll ? launch_kind<T, N, Q, true, true, kPointwise>(a, x, y, s)
+                                              : launch_kind<T, N, Q, true, false, kPointwise>(a, x, y, s);
+    if (a.field == kAffine) return a.gll ? launch_kind<T, N, Q, true, true, kAffine>(a, x, y, s)
+                                         : launch_kind<T, N, Q, true, false, kAffine>(a, x, y, s);
+    return a.gll ? launch_kind<T, N, Q, true, true, kSeparable>(a, x, y, s)
+                 : launch_kind<T, N, Q, true, false, kSeparable>(a, x, y, s);
   }
 }
 

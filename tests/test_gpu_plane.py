@@ -127,3 +127,52 @@ def test_diffusion_every_pair(n, q, basis, dtype):
 def test_diffusion_sizes_ranks_and_boundaries(sizes, periodic, rank):
     terms = [(1.5, {}), (0.3, {0: lambda s: s, 2: lambda s: 1.0 + s}), (0.2, {1: lambda s: s * s})][:rank]
     check_diffusion(space(sizes, 3, "L", periodic), 5, torch.float64, SeparableField(terms), 1.0 if rank == 2 else 0.0, 4.0)
+
+
+def pointwise_problem(fes, q, seed):
+    """Random per-point field (both signs on every face) as host arrays and as an operator."""
+    rng = np.random.default_rng(seed)
+    cell = rng.standard_normal((fes.mesh.num_cells, 3, q ** 3))
+    faces = [rng.standard_normal((f, q * q)) for f in G.face_counts(fes.mesh)]
+    dev = [torch.as_tensor(t, device="cuda") for t in (cell, *faces)]
+    return cell, faces, dev
+
+
+@pytest.mark.parametrize("sizes,periodic,bc", [((5, 3, 4), [True, False, True], "poly"), ((1, 1, 1), False, "zero"),
+                                               ((1, 5, 1), True, "none"), ((7, 5, 3), False, "none")], ids=str)
+@pytest.mark.parametrize("basis", ["L", "G"])
+@pytest.mark.parametrize("n,q", PAIRS)
+def test_pointwise_forward_transpose_and_gradient(n, q, basis, sizes, periodic, bc):
+    """The plane kernels of the per-point field: apply, adjoint and field gradient."""
+    fes = space(sizes, n - 1, basis, periodic)
+    ir, g = G.MakeIntegrationRule(q), bc_field(bc, 3)
+    cell, faces, dev = pointwise_problem(fes, q, 7)
+    op = G.MakeAdvectionOperator(fes, ir, G.PointwiseField(dev[0], dev[1:]), g)
+    u, r = G.fill_random(op.num_dofs, 21), G.fill_random(op.num_dofs, 22)
+    P = oracle.Problem(fes, ir, adv_coef=1.0, adv=(cell, faces), bc=g)
+    du, dr = torch.as_tensor(u, device="cuda"), torch.as_tensor(r, device="cuda")
+    nan = lambda t: torch.full_like(t, float("nan"))  # noqa: E731
+    y = op(du, nan(du))
+    assert rel_l2(y.cpu().numpy(), P.apply(u)) <= 1e-12
+    z = op.transpose(dr, nan(dr))
+    assert rel_l2(z.cpu().numpy(), P.apply_transpose(r)) <= 1e-12
+    dcell, dfaces = nan(dev[0]), [nan(t) for t in dev[1:]]
+    op.plan.grad_beta(0.7, du, dr, dcell, dfaces)
+    ref_cell, ref_faces = P.grad_beta(u, r, G.face_counts(fes.mesh))
+    assert rel_l2(dcell.cpu().numpy().ravel(), 0.7 * np.asarray(ref_cell).ravel()) <= 1e-12
+    for a in range(3):
+        want = 0.7 * np.asarray(ref_faces[a]).ravel()
+        got = dfaces[a].cpu().numpy().ravel()
+        assert np.linalg.norm(got - want) <= 1e-12 * max(np.linalg.norm(want), 1e-300)
+
+
+def test_pointwise_transpose_with_mass():
+    fes = space((4, 3, 5), 3, "L", [False, True, False])
+    ir = G.MakeIntegrationRule(5)
+    cell, faces, dev = pointwise_problem(fes, 5, 9)
+    sigma = sigma_field("poly", 3)
+    op = G.MakeMassAdvectionOperator(fes, ir, G.PointwiseField(dev[0], dev[1:]), sigma=sigma, mass_coef=0.6, adv_coef=-0.3)
+    r = G.fill_random(op.num_dofs, 5)
+    z = op.transpose(torch.as_tensor(r, device="cuda"), torch.empty(op.num_dofs, dtype=torch.float64, device="cuda"))
+    P = oracle.Problem(fes, ir, mass_coef=0.6, adv_coef=-0.3, sigma=sigma, adv=(cell, faces))
+    assert rel_l2(z.cpu().numpy(), P.apply_transpose(r)) <= 1e-12
