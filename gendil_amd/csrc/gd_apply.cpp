@@ -8,6 +8,7 @@
 #include "gd_dispatch.hpp"
 #include "gd_k3d_api.hpp"
 #include "gd_k3k_api.hpp"
+#include "gd_kron_api.hpp"
 #include "gd_n2k_api.hpp"
 #include "gd_padapt_api.hpp"
 #include "gd_padj_api.hpp"
@@ -74,7 +75,8 @@ template <typename T>
 int k3_choice(const gd_plan* plan, int N, bool adv, bool mass)
 {
   const int tuned = tuned_lanes(plan, N, sizeof(T));
-  if (tuned >= 0 && tuned != n2k::kVariant && tuned != pl::kVariant) return tuned;
+  if (tuned >= 0 && tuned != n2k::kVariant && tuned != pl::kVariant && tuned != kron::kVariant)
+    return tuned;
   if (N == 4 && k3k::available<T>(plan, 40, adv, mass)) return 16 + 40;
   const int ks = k3k::default_staged(N, sizeof(T));
   if (ks >= 0 && k3k::available<T>(plan, ks, adv, mass)) return 16 + ks;
@@ -93,6 +95,7 @@ bool k3_eligible(const gd_plan* plan, int choice, bool adv, bool mass)
 {
   if (choice == n2k::kVariant) return n2k::available<T>(plan, adv, mass);
   if (choice == pl::kVariant) return pl::available<T>(plan, adv, mass);
+  if (choice == kron::kVariant) return kron::available(plan, adv, mass);
   if (choice >= 16) return k3k::available<T>(plan, choice - 16, adv, mass);
   return k3::available<T>(plan, choice, adv, mass);
 }
@@ -133,6 +136,15 @@ int apply_impl(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, h
   if (plan->dim >= 4 && tuned_lanes(plan, 2, sizeof(T)) != 0 && n2k::available<T>(plan, adv, mass_coef != T(0))) {
     const int r = n2k::apply<T>(plan, mass_coef, adv_coef, x, y, s);
     if (r != GD_ERR_UNSUPPORTED) return r;
+  }
+  // 4D-6D sums of Kronecker products: the 6D p = 2 q = 3 phase-space apply of
+  // 19.7 M unknowns takes 163 us here and 2,650 us on the generic kernel
+  if (plan->dim >= 4) {
+    const int tuned = tuned_lanes(plan, 0, sizeof(T));
+    if (tuned == kron::kVariant || (tuned != 0 && kron::preferred(plan, adv, mass_coef != T(0)))) {
+      const int r = kron::apply<T>(plan, mass_coef, adv_coef, x, y, s);
+      if (r != GD_ERR_UNSUPPORTED) return r;
+    }
   }
   if (tuned_lanes(plan, 0, sizeof(T)) == pl::kVariant) {
     const int r = pl::apply<T>(plan, mass_coef, adv_coef, x, y, s);
@@ -249,7 +261,8 @@ int gd_plan_autotune(gd_plan* plan, int32_t precision_bytes, double mass_coef, d
   if (plan->padapt)
     for (int v = 0; v < gd::pa::num_variants(plan->dim); ++v) choices.push_back(v);
   else
-    choices = {0, 1, 2, 4, 17, 18, 20, 48, 49, 50, 51, 52, 53, 54, 55, 56, 57, gd::n2k::kVariant, gd::pl::kVariant};
+    choices = {0, 1, 2, 4, 17, 18, 20, 48, 49, 50, 51, 52, 53, 54, 55, 56, 57, gd::n2k::kVariant, gd::pl::kVariant,
+               gd::kron::kVariant};
   const int saved = *knob;
   double best = 1e300;
   int best_lanes = 0;
@@ -312,6 +325,12 @@ int gd_plan_query_variant(const gd_plan* plan, int32_t precision_bytes, double m
     if (plan->dim >= 4 && plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1] != 0 &&
         gd::n2k::available<T>(plan, adv, mass))
       return gd::n2k::kVariant;
+    if (plan->dim >= 4) {
+      const int tuned = plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1];
+      if (tuned == gd::kron::kVariant ? gd::kron::available(plan, adv, mass)
+                                      : tuned != 0 && gd::kron::preferred(plan, adv, mass))
+        return gd::kron::kVariant;
+    }
     if (plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1] == gd::pl::kVariant && gd::pl::available<T>(plan, adv, mass))
       return gd::pl::kVariant;
     const int choice = gd::k3_choice<T>(plan, N, adv, mass);
@@ -336,7 +355,8 @@ int gd_plan_set_variant(gd_plan* plan, int32_t precision_bytes, int32_t lanes)
     return GD_OK;
   }
   if (lanes != -1 && lanes != 0 && lanes != 1 && lanes != 2 && lanes != 4 && lanes != 17 && lanes != 18 &&
-      lanes != 20 && !(lanes >= 48 && lanes <= 57) && lanes != gd::n2k::kVariant && lanes != gd::pl::kVariant)
+      lanes != 20 && !(lanes >= 48 && lanes <= 57) && lanes != gd::n2k::kVariant && lanes != gd::pl::kVariant &&
+      lanes != gd::kron::kVariant)
     return fail(GD_ERR_INVALID, "gd_plan_set_variant: bad arguments");
   plan->tuned_k3_lanes[slot] = lanes;
   return GD_OK;

@@ -132,6 +132,10 @@ namespace k3k {
 struct State;
 void destroy_state(State* s);
 }  // namespace k3k
+namespace kron {
+struct State;
+void destroy_state(State* s);
+}  // namespace kron
 
 }  // namespace gd
 
@@ -185,6 +189,8 @@ struct gd_plan {
   mutable gd::pa::State* pa_state = nullptr;
   // factor tables of the Kronecker-factored 3D kernel (lazily built)
   mutable gd::k3k::State* k3k_state = nullptr;
+  // terms and matrices of the 4D-6D Kronecker kernel
+  mutable gd::kron::State* kron_state = nullptr;
   // basis tables at the mapped points of the subfaces of an h-nonconforming
   // interface (face operators), lazily built for the refinement ratios in
   // hmap_key

@@ -1,0 +1,384 @@
+// Host side of the 4D-6D Kronecker kernel: which coefficients it serves, the
+// terms and their matrices, launch.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <vector>
+
+#include "gd_kron.hpp"
+#include "gd_kron_api.hpp"
+
+namespace gd {
+namespace kron {
+
+// One term: matrices along a (and b), offsets into the device blobs; -1 none
+struct HostTerm {
+  int a = 0, b = 0, inflow = 0;
+  int64_t ta = -1, tb = -1, tf = -1;
+  double scale = 1.0;
+};
+
+struct State {
+  bool adv_ok = false, mass_ok = false;
+  std::vector<HostTerm> adv, mass;
+  double sigma_const = 0.0;  // sum of sigma's constant terms
+  int64_t mm = 0;            // offset of the mass matrix
+  // one allocation, kept from one set of coefficients to the next while they
+  // fit: the values in FP64, then in FP32
+  void* dev = nullptr;
+  size_t capacity = 0, words = 0;  // values
+  const double* f64() const { return static_cast<const double*>(dev); }
+  const float* f32() const { return reinterpret_cast<const float*>(f64() + words); }
+};
+
+void destroy_state(State* s)
+{
+  if (!s) return;
+  if (s->dev) (void)hipFree(s->dev);
+  delete s;
+}
+
+namespace {
+
+using Mat = std::vector<double>;  // n x n, row-major
+
+// inverse by Gauss-Jordan with partial pivoting, in extended precision
+Mat inverse(const Mat& a, int n)
+{
+  std::vector<long double> m((size_t)n * 2 * n, 0.0L);
+  for (int i = 0; i < n; ++i) {
+    for (int j = 0; j < n; ++j) m[i * 2 * n + j] = a[i * n + j];
+    m[i * 2 * n + n + i] = 1.0L;
+  }
+  for (int c = 0; c < n; ++c) {
+    int p = c;
+    for (int i = c + 1; i < n; ++i)
+      if (std::fabs((double)m[i * 2 * n + c]) > std::fabs((double)m[p * 2 * n + c])) p = i;
+    for (int j = 0; j < 2 * n; ++j) std::swap(m[c * 2 * n + j], m[p * 2 * n + j]);
+    const long double d = m[c * 2 * n + c];
+    for (int j = 0; j < 2 * n; ++j) m[c * 2 * n + j] /= d;
+    for (int i = 0; i < n; ++i) {
+      if (i == c) continue;
+      const long double f = m[i * 2 * n + c];
+      for (int j = 0; j < 2 * n; ++j) m[i * 2 * n + j] -= f * m[c * 2 * n + j];
+    }
+  }
+  Mat r((size_t)n * n);
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < n; ++j) r[i * n + j] = (double)m[i * 2 * n + n + j];
+  return r;
+}
+
+const Entry* find(const gd_plan* plan)
+{
+  List l{nullptr, 0};
+  if (plan->dim == 4) l = instances_d4();
+  else if (plan->dim == 5) l = instances_d5();
+  else if (plan->dim == 6) l = instances_d6();
+  for (int i = 0; i < l.n; ++i)
+    if (l.e[i].N == plan->desc.order + 1) return &l.e[i];
+  return nullptr;
+}
+
+// A field of at most one coordinate, as its axis (-1: constant) and its q + 2
+// samples per position along it
+struct OneAxis {
+  int axis = -1;
+  std::vector<double> v;  // axis < 0: one value
+};
+
+bool one_axis(const gd_plan* p, int c, const TableSet& ts, OneAxis& out)
+{
+  const int D = p->dim, q = ts.q;
+  if (p->beta_kind == GD_BETA_SEPARABLE) {
+    const HostField& f = p->beta_host[c];
+    double cst = 0.0;
+    int term = -1;
+    for (int r = 0; r < f.rank; ++r) {
+      int used = 0, ax = -1;
+      for (int d = 0; d < D; ++d)
+        if (f.offset[r][d] >= 0) {
+          ++used;
+          ax = d;
+        }
+      if (used == 0) cst += f.scale[r];
+      else if (used > 1 || term >= 0) return false;
+      else {
+        term = r;
+        out.axis = ax;
+      }
+    }
+    if (term < 0) {
+      out.v.assign(1, cst);
+      return true;
+    }
+    const int64_t n = p->desc.sizes[out.axis] * (q + 2);
+    out.v.resize(n);
+    for (int64_t i = 0; i < n; ++i) out.v[i] = cst + f.scale[term] * f.data[f.offset[term][out.axis] + i];
+    return true;
+  }
+  if (p->beta_kind != GD_BETA_AFFINE) return false;
+  for (int d = 0; d < D; ++d)
+    if (p->affA[c][d] != 0.0) {
+      if (out.axis >= 0) return false;
+      out.axis = d;
+    }
+  if (out.axis < 0) {
+    out.v.assign(1, p->affc[c]);
+    return true;
+  }
+  const int a = out.axis;
+  out.v.resize(p->desc.sizes[a] * (q + 2));
+  for (int64_t e = 0; e < p->desc.sizes[a]; ++e)
+    for (int k = 0; k < q + 2; ++k) {
+      const double xi = k < q ? ts.xq[k] : (k == q ? 0.0 : 1.0);
+      out.v[e * (q + 2) + k] =
+          p->affc[c] + p->affA[c][a] * ((p->desc.origin[a] + p->desc.h[a] * (double)e) + p->desc.h[a] * xi);
+    }
+  return true;
+}
+
+}  // namespace
+
+int refresh(const gd_plan* plan)
+{
+  if (!plan->kron_state) plan->kron_state = new State();
+  State& st = *plan->kron_state;
+  st.adv_ok = st.mass_ok = false;
+  st.adv.clear();
+  st.mass.clear();
+  st.sigma_const = 0.0;
+  const int D = plan->dim;
+  if (D < 4 || plan->padapt || plan->E >= (int64_t)1 << 31 || !find(plan)) return GD_OK;
+  const int n = plan->desc.order + 1, q = plan->desc.num_quad;
+  const TableSet* ts = find_tables(plan, n, q);
+  if (!ts || q < n) return GD_OK;  // M is singular with fewer points than nodes
+  auto gram = [&](const std::vector<double>& L, const double* f) {  // L^T W f B
+    Mat m((size_t)n * n, 0.0);
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j < n; ++j)
+        for (int k = 0; k < q; ++k) m[i * n + j] += ts->w[k] * (f ? f[k] : 1.0) * L[k * n + i] * ts->B[k * n + j];
+    return m;
+  };
+  const Mat M = gram(ts->B, nullptr), Mi = inverse(M, n);
+  std::vector<double> blob;
+  auto put = [&](const Mat& m) {
+    const int64_t at = (int64_t)blob.size();
+    blob.insert(blob.end(), m.begin(), m.end());
+    return at;
+  };
+  auto times = [&](const Mat& m) {  // M^-1 m, m with n rows
+    const int cols = (int)m.size() / n;
+    Mat r(m.size(), 0.0);
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j < cols; ++j) {
+        long double s = 0.0L;
+        for (int k = 0; k < n; ++k) s += (long double)Mi[i * n + k] * m[k * cols + j];
+        r[i * cols + j] = (double)s;
+      }
+    return r;
+  };
+  st.mm = put(M);
+  // factor matrices M^-1 B^T W f B per position along an axis
+  auto factor = [&](int axis, const double* v, double scale) {
+    const int64_t at = (int64_t)blob.size();
+    for (int64_t e = 0; e < plan->desc.sizes[axis]; ++e) {
+      Mat f(q);
+      for (int k = 0; k < q; ++k) f[k] = scale * v[e * (q + 2) + k];
+      put(times(gram(ts->B, f.data())));
+    }
+    return at;
+  };
+
+  // ---- sigma ----
+  st.mass_ok = true;
+  for (int r = 0; r < plan->sigma_host.rank && st.mass_ok; ++r) {
+    const HostField& f = plan->sigma_host;
+    std::vector<int> ax;
+    for (int d = 0; d < D; ++d)
+      if (f.offset[r][d] >= 0) ax.push_back(d);
+    if (ax.empty()) {
+      st.sigma_const += f.scale[r];
+      continue;
+    }
+    if (ax.size() > 2 || st.mass.size() == 4) {
+      st.mass_ok = false;
+      break;
+    }
+    HostTerm t;
+    t.a = ax[0];
+    t.ta = factor(ax[0], f.data.data() + f.offset[r][ax[0]], f.scale[r]);
+    t.b = ax.size() > 1 ? ax[1] : (ax[0] == 0 ? 1 : 0);
+    if (ax.size() > 1) t.tb = factor(ax[1], f.data.data() + f.offset[r][ax[1]], 1.0);
+    st.mass.push_back(t);
+  }
+
+  // ---- advection ----
+  st.adv_ok = plan->beta_set && (plan->bc_mode == GD_BC_NONE || plan->bc_host.rank == 0 ||
+                                 (plan->bc_host.rank == 1 && plan->bc_host.scale[0] == 0.0));
+  for (int c = 0; c < D && st.adv_ok; ++c) {
+    OneAxis f;
+    if (!one_axis(plan, c, *ts, f)) {
+      st.adv_ok = false;
+      break;
+    }
+    // one sign on every face point: the rule points along the field's axis, or
+    // its ends where that is the normal
+    bool pos = false, neg = false, zero = true;
+    if (f.axis < 0) {
+      pos = f.v[0] > 0.0;
+      neg = f.v[0] < 0.0;
+      zero = f.v[0] == 0.0;
+    } else {
+      for (size_t i = 0; i < f.v.size(); ++i) {
+        const int k = (int)(i % (q + 2));
+        zero = zero && f.v[i] == 0.0;
+        if (f.axis == c ? k < q : k >= q) continue;
+        pos |= f.v[i] > 0.0;
+        neg |= f.v[i] < 0.0;
+      }
+    }
+    for (double v : f.v) st.adv_ok = st.adv_ok && std::isfinite(v);
+    if ((pos && neg) || !st.adv_ok) {
+      st.adv_ok = false;
+      break;
+    }
+    if (zero) continue;
+    const bool per = plan->desc.periodic[c];
+    const int64_t Mc = plan->desc.sizes[c];
+    HostTerm t;
+    t.a = c;
+    t.b = f.axis >= 0 && f.axis != c ? f.axis : (c == 0 ? 1 : 0);
+    t.inflow = neg ? -1 : 1;
+    t.scale = 1.0 / plan->desc.h[c];
+    Mat fv;
+    t.ta = (int64_t)blob.size();
+    for (int64_t e = 0; e < Mc; ++e) {
+      const double* v = f.axis == c ? f.v.data() + e * (q + 2) : nullptr;
+      const double cst = f.axis < 0 ? f.v[0] : 1.0;
+      Mat m = gram(ts->Gb, v);
+      for (double& s : m) s *= -cst;
+      // own face at the outflow end: there with a neighbour or inflow data
+      const bool edge = !per && (neg ? e == 0 : e == Mc - 1);
+      if (!(edge && plan->bc_mode == GD_BC_NONE)) {
+        const std::vector<double>& be = neg ? ts->b0 : ts->b1;
+        const double bo = (v ? v[neg ? q : q + 1] : 1.0) * cst * (neg ? -1.0 : 1.0);
+        for (int i = 0; i < n; ++i)
+          for (int j = 0; j < n; ++j) m[i * n + j] += bo * be[i] * be[j];
+      }
+      put(times(m));
+      // inflow end: -beta b0 (lower face) or +beta b1 (upper face) on the neighbour's trace
+      const double bi = (v ? v[neg ? q + 1 : q] : 1.0) * cst * (neg ? 1.0 : -1.0);
+      Mat col(n);
+      for (int i = 0; i < n; ++i) col[i] = bi * (neg ? ts->b1[i] : ts->b0[i]);
+      const Mat fc = times(col);
+      fv.insert(fv.end(), fc.begin(), fc.end());
+    }
+    t.tf = put(fv);
+    if (f.axis >= 0 && f.axis != c) t.tb = factor(f.axis, f.v.data(), 1.0);
+    st.adv.push_back(t);
+  }
+  if (!st.adv_ok && !st.mass_ok) return GD_OK;
+  st.words = blob.size();
+  if (st.words > st.capacity) {
+    if (st.dev) (void)hipFree(st.dev);
+    st.dev = nullptr;
+    st.capacity = 0;
+    const size_t want = std::max<size_t>(2 * st.words, 4096);
+    if (hipMalloc(&st.dev, want * (sizeof(double) + sizeof(float))) != hipSuccess) {
+      st.adv_ok = st.mass_ok = false;
+      return fail(GD_ERR_ALLOC, "Kronecker tables: device allocation failed");
+    }
+    st.capacity = want;
+  }
+  std::vector<char> host(st.words * (sizeof(double) + sizeof(float)));
+  std::memcpy(host.data(), blob.data(), st.words * sizeof(double));
+  float* h32 = reinterpret_cast<float*>(host.data() + st.words * sizeof(double));
+  for (size_t i = 0; i < st.words; ++i) h32[i] = (float)blob[i];
+  const hipError_t err = hipMemcpy(st.dev, host.data(), host.size(), hipMemcpyHostToDevice);
+  if (err != hipSuccess) {
+    st.adv_ok = st.mass_ok = false;
+    return hip_fail(err, "hipMemcpy");
+  }
+  return GD_OK;
+}
+
+bool available(const gd_plan* plan, bool adv, bool mass)
+{
+  const State* st = plan->kron_state;
+  return st && (st->adv_ok || st->mass_ok) && (!adv || st->adv_ok) && (!mass || st->mass_ok);
+}
+
+bool preferred(const gd_plan* plan, bool adv, bool mass)
+{
+  // a handful of elements (unit tests, debugging runs) stay on the generic
+  // kernel, which takes the quadrature as it is written
+  return plan->E > 64 && available(plan, adv, mass);
+}
+
+template <typename T>
+int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStream_t s)
+{
+  const bool adv = adv_coef != T(0), mass = mass_coef != T(0);
+  if (!available(plan, adv, mass)) return GD_ERR_UNSUPPORTED;
+  const Entry* en = find(plan);
+  const State& st = *plan->kron_state;
+  const TableSet* ts = find_tables(plan, plan->desc.order + 1, plan->desc.num_quad);
+  const int D = plan->dim, n = plan->desc.order + 1;
+  Args<T> a;
+  const T* base;
+  const Tables1D<T>* tab;
+  if constexpr (std::is_same_v<T, double>) {
+    base = st.f64();
+    tab = &ts->t64;
+  } else {
+    base = st.f32();
+    tab = &ts->t32;
+  }
+  a.E = (int)plan->E;
+  a.periodic_mask = 0;
+  double detJ = 1.0;
+  for (int d = 0; d < D; ++d) {
+    a.M[d] = (int)plan->desc.sizes[d];
+    if (d < 5) a.dv[d] = pl::fast_div(a.M[d]);
+    if (plan->desc.periodic[d]) a.periodic_mask |= 1 << d;
+    detJ *= plan->desc.h[d];
+  }
+  a.km = mass ? (T)((double)mass_coef * detJ * st.sigma_const) : T(0);
+  a.Mm = base + st.mm;
+  a.b0 = tab->b0;
+  a.b1 = tab->b1;
+  a.nterms = 0;
+  auto add = [&](const HostTerm& h, double coef) {
+    Term<T>& t = a.t[a.nterms];
+    a.coef[a.nterms++] = (T)(coef * detJ * h.scale);
+    t.a = h.a;
+    t.b = h.b;
+    t.inflow = h.inflow;
+    t.ta = base + h.ta;
+    t.tb = h.tb >= 0 ? base + h.tb : nullptr;
+    t.tf = h.tf >= 0 ? base + h.tf : nullptr;
+    int k = 0, st_ = 1;
+    for (int d = 0; d < D; ++d) {
+      if (d == h.a) t.stride[D - 2] = st_;
+      else if (d == h.b) t.stride[D - 1] = st_;
+      else t.stride[k++] = st_;
+      st_ *= n;
+    }
+  };
+  if (adv)
+    for (const HostTerm& h : st.adv) add(h, (double)adv_coef);
+  if (mass)
+    for (const HostTerm& h : st.mass) add(h, (double)mass_coef);
+  const bool gll = plan->desc.basis == GD_BASIS_GLL;
+  if constexpr (std::is_same_v<T, double>) return en->f64(a, gll, x, y, s);
+  else return en->f32(a, gll, x, y, s);
+}
+
+template int apply<double>(const gd_plan*, double, double, const double*, double*, hipStream_t);
+template int apply<float>(const gd_plan*, float, float, const float*, float*, hipStream_t);
+
+}  // namespace kron
+}  // namespace gd

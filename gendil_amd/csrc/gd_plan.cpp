@@ -13,6 +13,7 @@
 
 #include "gd_internal.hpp"
 #include "gd_k3k_api.hpp"
+#include "gd_kron_api.hpp"
 #include "gd_padapt_api.hpp"
 
 namespace gd {
@@ -356,6 +357,7 @@ int commit_coefficients(gd_plan* p, bool fields)
     if (int rc = upload_fields(p)) return rc;
   }
   if (int rc = k3k::refresh(p)) return rc;
+  if (int rc = kron::refresh(p)) return rc;
   return pa::refresh(p);
 }
 
@@ -439,6 +441,7 @@ gd_plan::~gd_plan()
   gd::free_fields(this);
   gd::pa::destroy_state(pa_state);
   gd::k3k::destroy_state(k3k_state);
+  gd::kron::destroy_state(kron_state);
   if (hmap_dev) (void)hipFree(hmap_dev);
 }
 
@@ -551,6 +554,7 @@ int gd_plan_create(const gd_desc* desc, gd_plan** out)
   gd::copy_sep(p, nullptr, p->bc_host, 0.0);
   int rc = gd::upload_fields(p);
   if (rc == GD_OK) rc = gd::k3k::refresh(p);
+  if (rc == GD_OK) rc = gd::kron::refresh(p);
   if (rc == GD_OK) rc = gd::pa::refresh(p);
   if (rc != GD_OK) {
     delete p;

@@ -188,7 +188,7 @@ class Plan:
         a time), 56 / 57 (streaming form: one wave per block, persistent; 56 one tile buffer and two
         waves per SIMD, 57 two tile buffers with the next tile's copies in flight), 64 (4D-6D, order 1,
         constant coefficients: two-node Kronecker kernel), 72 (3D, any basis, rule and separable or affine
-        field: plane kernel);
+        field: plane kernel), 73 (4D-6D, one-axis field of one sign per component: Kronecker kernel);
         p-adaptive plans: the layout index."""
         nbytes = 8 if dtype == torch.float64 else 4
         L.check(L.lib().gd_plan_set_variant(self.handle, nbytes, lanes), "gd_plan_set_variant")

@@ -232,7 +232,8 @@ int gd_plan_autotune(gd_plan* plan, int32_t precision_bytes, double mass_coef, d
 /* Pin a variant: -1 (default); uniform plans 0 (generic), 1, 2 or 4 lanes
  * (register kernel), 17, 18 or 20 (Kronecker kernel), 48..55 (LDS-staged
  * Kronecker kernel), 56 or 57 (streaming Kronecker kernel), 64 (two-node
- * Kronecker kernel, 4D-6D), 72 (plane kernel, 3D); p-adaptive plans the variant index as reported by
+ * Kronecker kernel, 4D-6D), 72 (plane kernel, 3D),
+ * 73 (Kronecker kernel, 4D-6D); p-adaptive plans the variant index as reported by
  * gd_plan_autotune.  A pinned variant that does not serve a later apply
  * falls back to the default for that apply. */
 int gd_plan_set_variant(gd_plan* plan, int32_t precision_bytes, int32_t lanes);
