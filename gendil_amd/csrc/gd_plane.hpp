@@ -670,7 +670,9 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
       T* r = rec + (el * PL + kz) * PITCH;
       const T* sm = smp + el * a.spitch;
       const T wz = ((GPtr<T>)a.w)[kz];
-      T v[Q][Q], xo[2][Q];
+      T v[Q][Q], xo[2][Q], b[Q][Q];
+      // a pointwise field's first plane is on its way during the interpolation
+      if constexpr (ADV && FIELD == kPointwise) beta_at(0, e, sub, smp, kz, wz, b);
       {
         T u[N][N];
 #pragma unroll
@@ -697,7 +699,6 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
 #pragma unroll
           for (int i = 0; i < N; ++i) out[m][i] = mad(tab(k, m), g[i], out[m][i]);
       };
-      T b[Q][Q];
       if constexpr (ADV) {
         const bool none = a.bc_none;
         // upwind flux of one face point: c = adv_coef detJ / h times the
@@ -732,7 +733,7 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
               pin(fx[s]);
             }
           }
-          beta_at(0, e, sub, sm, kz, wz, b);
+          if constexpr (FIELD != kPointwise) beta_at(0, e, sub, sm, kz, wz, b);
 #pragma unroll
           for (int k = 0; k < Q; ++k) {
             T f[Q], g[N];
