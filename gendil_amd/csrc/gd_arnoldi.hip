@@ -2,36 +2,41 @@
 //
 // One iteration k (basis vectors V_0..V_k stored with scales s_j, true vector
 // v_j = s_j V_j, and W = V_{k+1} holding K V_k) is three fused passes over the
-// basis, each followed by a one-block kernel that sums the block partials in a
-// fixed order (deterministic) and finishes the pass's scalar work:
+// basis:
 //   pass A: h1_j = s_j <V_j, W>                         (classical GS)
 //   pass B: W -= sum_j s_j h1_j V_j, then h2_j = s_j <V_j, W>, ||W||^2
 //           (re-orthogonalisation, the "twice is enough" CGS2 step)
 //   pass C: Z = (W - sum_j s_j h2_j V_j) / p with p^2 = ||W||^2 - sum_j h2_j^2
 //           (Pythagoras), stored as V_{k+1}; nu = ||Z|| exactly; s_{k+1} = 1/nu
-// and the finishing kernel of pass C forms the Hessenberg column
-// H_{jk} = s_k (h1_j + h2_j), H_{k+1,k} = s_k p nu, applies the previous Givens
-// rotations and forms the new one (gmres.hpp:170-210).  Stored vectors are
-// kept at unit norm (up to rounding), so the operator is applied with scale 1
-// and FP32 bases cannot drift out of range.
+// then the Hessenberg column H_{jk} = s_k (h1_j + h2_j), H_{k+1,k} = s_k p nu is
+// formed and rotated by the previous Givens rotations and a new one
+// (gmres.hpp:170-210).  Stored vectors are kept at unit norm (up to rounding),
+// so the operator is applied with scale 1 and FP32 bases cannot drift out of
+// range.
+//
+// The passes are bandwidth-bound (FP32, 2.1 M values, 30 vectors: 252 MB in
+// ~47 us), so what is left to save is the time between them.  Each pass leaves
+// one partial per block and column; the next pass sums them in its own prologue,
+// every block for itself in the same fixed order (at most 256 partials of 33
+// columns or 512 of 9: ~64 KB from L2), and pass C's column is finished by one
+// wave of the next step's pass A (or by a one-wave kernel before the cycle's
+// update).  Against one-block finishing kernels between the passes (4-6 us each
+// and a launch gap): the 32^3, p = 3 implicit step in mixed precision (47 cycles of
+// 30) 160.6 -> 145.4 ms.  Walking every second pass downwards for the L2 and
+// loading the first packs before the sums measured the same, with spills.
 //
 // The residual estimate |g_{k+1}| goes to the caller's pointer (pinned host
 // memory, so a host loop can poll it with no copy or event in the stream) from
-// the first block of the next kernel on the workspace (the next step's pass A
-// or the cycle's update), early in a kernel that still runs for a while: a
-// store to host memory at the end of a kernel holds the kernel's completion
-// for the bus round trip.
-//
-// The reductions end in separate one-block kernels rather than in the last
-// block of each pass: a device-scope fence per block (needed to publish the
-// partials across the XCDs' L2 caches) cost more than the extra launch.
+// the first block of the next kernel on the workspace that runs on for a while
+// (the next step's pass A or the cycle's update): a store to host memory at the
+// end of a kernel holds the kernel's completion for the bus round trip.
 //
 // FP32 bases are read 16 bytes per lane (4 values) where the basis and its
 // leading dimension are 16-byte aligned (pass B, which keeps every loaded
 // value live, 8 bytes); FP64 bases one value per lane, which measured as fast.
 //
-// The cycle end solves the triangular system H y = g in every block (k <= 32,
-// cheap) and adds x += sum_j s_j y_j V_j in FP64.
+// The cycle end solves the triangular system H y = g in one wave (with the last
+// column's finish) and adds x += sum_j s_j y_j V_j in FP64.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -43,24 +48,29 @@
 namespace gd {
 namespace arnoldi {
 
-using red::kFinThreads;
-using red::kMaxBlocks;
-using red::kThreads;
+constexpr int kThreads = 512;       // two waves per SIMD: up to 256 registers for the loads in flight
 constexpr int kMaxM = 32;           // restart length
-constexpr int kStride = kMaxM + 2;  // partial columns per block: k+1 dots + norm
-static_assert(kFinThreads == kMaxBlocks, "one block's partials per finishing thread");
+constexpr int kStride = kMaxM + 1;  // partial columns per block: k+1 dots + norm
+constexpr int kMaxBlocks = 512;     // partials per column
+// blocks of a pass over KK vectors: two per CU while there are few loads per
+// thread (and few columns to sum), else one
+constexpr int max_blocks(int KK) { return KK <= 8 ? kMaxBlocks : kMaxBlocks / 2; }
 
 struct Workspace {
   double H[kMaxM][kMaxM + 1];  // column k, rows 0..k+1 (rotated)
   double cs[kMaxM], sn[kMaxM];
   double g[kMaxM + 1];
   double s[kMaxM + 1];
-  double c[kMaxM];   // coefficients on the stored vectors for the next update pass
+  double c[kMaxM];   // coefficients on the stored vectors for the cycle's update
   double h1[kMaxM];  // accumulated true GS coefficients of the current column
-  double pnorm, pinv;
-  double* pending;   // caller pointer still owed the last residual estimate
+  double pnorm;
+  int owed, owed_blocks;  // columns whose rotation is still to be formed (its number + 1, or 0), partials in pc
+  double* owed_out;       // where that column's residual estimate goes
+  double* pending;        // caller pointer still owed the last residual estimate
   double pending_value;
-  double partial[kStride][kMaxBlocks];  // [column][block]: a column is contiguous
+  double pa[kMaxM][kMaxBlocks];  // [column][block]: a column is contiguous
+  double pb[kStride][kMaxBlocks];
+  double pc[kMaxBlocks];
 };
 
 // W values of one vector, loaded or stored as one access of up to 16 bytes
@@ -82,18 +92,111 @@ __device__ __forceinline__ void st(T* p, const Pack<T, W>& v)
   *reinterpret_cast<Pack<T, W>*>(p) = v;
 }
 
-using red::grid_for;
-
-template <int K>
-__device__ __forceinline__ void store_block_partials(const double (&acc)[K], Workspace* ws)
+// One pack per thread until the grid is at its largest: a small basis spread
+// over all CUs (four packs per thread left 28^3 p = 2 in FP32 on 72 of them:
+// 37.2 ms a solve against 29.0; start 33.7).
+inline int grid_for(int64_t n, int w, int most)
 {
-  red::store_block_partials<K>(acc, ws->partial);
+  const int64_t per = (int64_t)kThreads * w;
+  const int64_t b = (n + per - 1) / per;
+  return (int)(b < 1 ? 1 : (b > most ? most : b));
+}
+
+// Lane i's value, i the same in the whole wave.
+__device__ __forceinline__ double lane_value(double v, int i)
+{
+  union {
+    double d;
+    int w[2];
+  } u{v};
+  u.w[0] = __builtin_amdgcn_readlane(u.w[0], i);
+  u.w[1] = __builtin_amdgcn_readlane(u.w[1], i);
+  return u.d;
 }
 
 template <int K>
-__device__ __forceinline__ void sum_partials(const Workspace* ws, int nblk, double* col)
+__device__ __forceinline__ void store_block_partials(const double (&acc)[K], double (*partial)[kMaxBlocks])
 {
-  red::sum_partials<K>(ws->partial, nblk, col);
+  __shared__ double row[K];
+  red::block_sum<kThreads, K>(acc, row);
+  for (int j = threadIdx.x; j < K; j += kThreads) partial[j][blockIdx.x] = row[j];
+}
+
+// col[j] = sum over nblk <= MAXB partials of column j, j < K: TPC threads per
+// column, all their loads in flight together, then a shuffle sum; a fixed order
+// for a given grid.  Visible to every thread on return.
+template <int K, int MAXB>
+__device__ __forceinline__ void sum_columns(const double (*partial)[kMaxBlocks], int nblk, double* col)
+{
+  constexpr int TPC = K <= 8 ? 64 : K <= 16 ? 32 : 16;
+  constexpr int CPP = kThreads / TPC;  // columns per round
+  constexpr int PER = MAXB / TPC;      // partials per thread
+  const int lane = threadIdx.x % TPC, c0 = threadIdx.x / TPC;
+#pragma unroll
+  for (int r = 0; r < (K + CPP - 1) / CPP; ++r) {
+    const int j = c0 + r * CPP;
+    if (j < K) {  // uniform over each group of TPC threads; the shuffles stay inside it
+      const double* cp = partial[j];
+      double v[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int bb = lane + TPC * i;
+        const double x = cp[bb < nblk ? bb : nblk - 1];
+        v[i] = bb < nblk ? x : 0.0;
+      }
+      double sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) sum += v[i];
+#pragma unroll
+      for (int off = TPC / 2; off > 0; off >>= 1) sum += __shfl_down(sum, off, TPC);
+      if (lane == 0) col[j] = sum;
+    }
+  }
+  __syncthreads();
+}
+
+// One whole wave: the owed column of the Hessenberg matrix (row j in lane j),
+// its Givens rotation and residual estimate (left pending).
+__device__ __forceinline__ void finish_column(Workspace* __restrict__ ws)
+{
+  const int owed = ws->owed;
+  if (owed == 0) return;
+  const int k = owed - 1, lane = threadIdx.x & 63, nblk = ws->owed_blocks;
+  double part = 0.0;
+#pragma unroll
+  for (int i = 0; i < kMaxBlocks / 64; ++i) {
+    const int bb = lane + 64 * i;
+    const double x = ws->pc[bb < nblk ? bb : nblk - 1];
+    part += bb < nblk ? x : 0.0;
+  }
+  const double sk = ws->s[k];
+  const double c_l = lane < k ? ws->cs[lane] : 1.0, s_l = lane < k ? ws->sn[lane] : 0.0;
+  double h = lane <= k ? sk * ws->h1[lane < kMaxM ? lane : 0] : 0.0;
+  const double nu = sqrt(lane_value(red::wave_sum(part), 0));
+  if (lane == owed) h = sk * ws->pnorm * nu;
+  double carry = lane_value(h, 0), out = 0.0;
+  for (int i = 0; i < k; ++i) {
+    const double b = lane_value(h, i + 1), c = lane_value(c_l, i), sn = lane_value(s_l, i);
+    if (lane == i) out = c * carry + sn * b;
+    carry = -sn * carry + c * b;
+  }
+  const double a = carry, b = lane_value(h, owed);
+  const double rho = hypot(a, b);
+  const double cs = rho > 0.0 ? a / rho : 1.0, sn = rho > 0.0 ? b / rho : 0.0;
+  if (lane == k) out = rho;
+  if (lane <= owed) ws->H[k][lane] = out;
+  if (lane == 0) {
+    ws->s[owed] = nu > 0.0 ? 1.0 / nu : 0.0;
+    ws->cs[k] = cs;
+    ws->sn[k] = sn;
+    const double gk = ws->g[k];
+    const double g1 = -sn * gk;
+    ws->g[owed] = g1;
+    ws->g[k] = cs * gk;
+    ws->pending = ws->owed_out;
+    ws->pending_value = fabs(g1);
+    ws->owed = 0;
+  }
 }
 
 __device__ __forceinline__ void publish_pending(Workspace* ws) { red::publish_pending(&ws->pending, &ws->pending_value); }
@@ -109,7 +212,10 @@ template <typename TV, int KK, int W>
 __global__ void __launch_bounds__(kThreads) k_pass_a(int64_t n, const TV* __restrict__ V, int64_t ldv,
                                                      Workspace* __restrict__ ws)
 {
-  publish_pending(ws);
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    finish_column(ws);
+    publish_pending(ws);
+  }
   const TV* __restrict__ w = V + (int64_t)KK * ldv;
   double acc[KK];
 #pragma unroll
@@ -130,31 +236,29 @@ __global__ void __launch_bounds__(kThreads) k_pass_a(int64_t n, const TV* __rest
 #pragma unroll
     for (int j = 0; j < KK; ++j) acc[j] += (double)V[j * ldv + i] * wi;
   }
-  store_block_partials<KK>(acc, ws);
+  store_block_partials<KK>(acc, ws->pa);
 }
 
-// h1_j = s_j <V_j, W>, c_j = s_j h1_j.
-template <int KK>
-__global__ void __launch_bounds__(kFinThreads) k_fin_a(int nblk, Workspace* __restrict__ ws)
-{
-  __shared__ double col[KK];
-  sum_partials<KK>(ws, nblk, col);
-  for (int j = threadIdx.x; j < KK; j += kFinThreads) {
-    const double h = ws->s[j] * col[j];
-    ws->h1[j] = h;
-    ws->c[j] = ws->s[j] * h;
-  }
-}
-
-// Pass B: W -= sum_j c_j V_j; partial row = <V_j, W_new>, ||W_new||^2.
+// Pass B: h1_j = s_j <V_j, W>, c_j = s_j h1_j; W -= sum_j c_j V_j; partial row = <V_j, W_new>, ||W_new||^2.
 template <typename TV, int KK, int W>
 __global__ void __launch_bounds__(kThreads) k_pass_b(int64_t n, TV* __restrict__ V, int64_t ldv,
                                                      Workspace* __restrict__ ws)
 {
   TV* __restrict__ w = V + (int64_t)KK * ldv;
+  __shared__ double col[KK];
+  sum_columns<KK, max_blocks(KK)>(ws->pa, gridDim.x, col);
+  double c_l = 0.0;
+  {
+    const int j = threadIdx.x & 63;
+    if (j < KK) {
+      const double sj = ws->s[j], h = sj * col[j];
+      if (blockIdx.x == 0 && threadIdx.x < 64) ws->h1[j] = h;
+      c_l = sj * h;
+    }
+  }
   double cj[KK];
 #pragma unroll
-  for (int j = 0; j < KK; ++j) cj[j] = ws->c[j];
+  for (int j = 0; j < KK; ++j) cj[j] = lane_value(c_l, j);
   double acc[KK + 1];
 #pragma unroll
   for (int j = 0; j <= KK; ++j) acc[j] = 0.0;
@@ -199,45 +303,46 @@ __global__ void __launch_bounds__(kThreads) k_pass_b(int64_t n, TV* __restrict__
     for (int j = 0; j < KK; ++j) acc[j] += v[j] * wr;
     acc[KK] += wr * wr;
   }
-  store_block_partials<KK + 1>(acc, ws);
+  store_block_partials<KK + 1>(acc, ws->pb);
 }
 
-// h2_j = s_j <V_j, W>, h1_j += h2_j, c_j = s_j h2_j,
-// p = sqrt(||W||^2 - sum_j h2_j^2).
-template <int KK>
-__global__ void __launch_bounds__(kFinThreads) k_fin_b(int nblk, Workspace* __restrict__ ws)
-{
-  __shared__ double col[KK + 1];
-  __shared__ double h2sq[KK];
-  sum_partials<KK + 1>(ws, nblk, col);
-  for (int j = threadIdx.x; j < KK; j += kFinThreads) {
-    const double h2 = ws->s[j] * col[j];
-    ws->h1[j] += h2;
-    ws->c[j] = ws->s[j] * h2;
-    h2sq[j] = h2 * h2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double ss = 0.0;
-#pragma unroll
-    for (int j = 0; j < KK; ++j) ss += h2sq[j];
-    const double p2 = col[KK] - ss;
-    const double p = p2 > 0.0 ? sqrt(p2) : 0.0;
-    ws->pnorm = p;
-    ws->pinv = p > 0.0 ? 1.0 / p : 0.0;
-  }
-}
-
-// Pass C: Z = (W - sum_j c_j V_j) / p stored as V_KK; partial = ||Z||^2.
+// Pass C: h2_j = s_j <V_j, W>, h1_j += h2_j, c_j = s_j h2_j,
+// p = sqrt(||W||^2 - sum_j h2_j^2); Z = (W - sum_j c_j V_j) / p stored as V_KK;
+// partial = ||Z||^2.
 template <typename TV, int KK, int W>
 __global__ void __launch_bounds__(kThreads) k_pass_c(int64_t n, TV* __restrict__ V, int64_t ldv,
-                                                     Workspace* __restrict__ ws)
+                                                     Workspace* __restrict__ ws, double* resid_out)
 {
   TV* __restrict__ w = V + (int64_t)KK * ldv;
-  const double pinv = ws->pinv;
+  __shared__ double col[KK + 1];
+  sum_columns<KK + 1, max_blocks(KK)>(ws->pb, gridDim.x, col);
+  double c_l = 0.0, h2 = 0.0;
+  const int lane = threadIdx.x & 63;
+  if (lane < KK) {
+    const double sj = ws->s[lane];
+    h2 = sj * col[lane];
+    c_l = sj * h2;
+  }
   double cj[KK];
+  double ss = 0.0;
 #pragma unroll
-  for (int j = 0; j < KK; ++j) cj[j] = ws->c[j];
+  for (int j = 0; j < KK; ++j) {
+    cj[j] = lane_value(c_l, j);
+    const double hj = lane_value(h2, j);
+    ss += hj * hj;
+  }
+  const double p2 = col[KK] - ss;
+  const double p = p2 > 0.0 ? sqrt(p2) : 0.0;
+  const double pinv = p > 0.0 ? 1.0 / p : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    if (lane < KK) ws->h1[lane] += h2;
+    if (lane == 0) {
+      ws->pnorm = p;
+      ws->owed = KK;
+      ws->owed_blocks = gridDim.x;
+      ws->owed_out = resid_out;
+    }
+  }
   double acc[1] = {0.0};
   const int64_t nv = n / W, stride = (int64_t)gridDim.x * kThreads;
   const int64_t t0 = (int64_t)blockIdx.x * kThreads + threadIdx.x;
@@ -270,51 +375,7 @@ __global__ void __launch_bounds__(kThreads) k_pass_c(int64_t n, TV* __restrict__
     const double zr = (double)zt;
     acc[0] += zr * zr;
   }
-  store_block_partials<1>(acc, ws);
-}
-
-// Column k = KK - 1 of the Hessenberg matrix and its Givens rotation; the
-// residual estimate |g_{k+1}| is left for the next kernel to publish.
-template <int KK>
-__global__ void __launch_bounds__(kFinThreads) k_fin_c(int nblk, Workspace* __restrict__ ws,
-                                                       double* __restrict__ resid_out)
-{
-  constexpr int k = KK - 1;
-  __shared__ double col[1];
-  __shared__ double hc[KK + 1];
-  sum_partials<1>(ws, nblk, col);
-  const double sk = ws->s[k];
-  for (int j = threadIdx.x; j <= k; j += kFinThreads) hc[j] = sk * ws->h1[j];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double nu = sqrt(col[0]);
-    ws->s[k + 1] = nu > 0.0 ? 1.0 / nu : 0.0;
-    double h[KK + 1];
-#pragma unroll
-    for (int j = 0; j <= k; ++j) h[j] = hc[j];
-    h[k + 1] = sk * ws->pnorm * nu;
-#pragma unroll
-    for (int i = 0; i < k; ++i) {
-      const double a = h[i], b = h[i + 1], c = ws->cs[i], sn = ws->sn[i];
-      h[i] = c * a + sn * b;
-      h[i + 1] = -sn * a + c * b;
-    }
-    const double a = h[k], b = h[k + 1];
-    const double rho = hypot(a, b);
-    const double cs = rho > 0.0 ? a / rho : 1.0, sn = rho > 0.0 ? b / rho : 0.0;
-    ws->cs[k] = cs;
-    ws->sn[k] = sn;
-    h[k] = rho;
-    h[k + 1] = 0.0;
-#pragma unroll
-    for (int j = 0; j <= k + 1; ++j) ws->H[k][j] = h[j];
-    const double gk = ws->g[k];
-    const double g1 = -sn * gk;
-    ws->g[k + 1] = g1;
-    ws->g[k] = cs * gk;
-    ws->pending = resid_out;
-    ws->pending_value = fabs(g1);
-  }
+  store_block_partials<1>(acc, &ws->pc);
 }
 
 // Cycle start: g = beta e_0, s_0 = s0, no residual estimate owed (the
@@ -326,32 +387,37 @@ __global__ void k_begin(double beta, double s0, Workspace* __restrict__ ws)
   if (t == 0) {
     ws->s[0] = s0;
     ws->pending = nullptr;
+    ws->owed = 0;
   }
 }
 
-// Cycle end: y = H(0:k,0:k)^{-1} g(0:k) in every block, x += sum_j s_j y_j V_j.
+// Cycle end, one wave: the last column, then y = H(0:k,0:k)^{-1} g(0:k) by
+// columns (row j in lane j) and c_j = s_j y_j.
+__global__ void __launch_bounds__(64) k_solve_cycle(int k, Workspace* __restrict__ ws)
+{
+  finish_column(ws);
+  __threadfence_block();
+  const int lane = threadIdx.x;
+  const int row = lane < k ? lane : 0;
+  double acc = ws->g[row];
+  for (int i = k - 1; i >= 0; --i) {
+    const double hij = ws->H[i][row];
+    const double y = lane_value(acc, i) / lane_value(hij, i);
+    if (lane == i) acc = y;
+    else if (lane < i) acc -= hij * y;
+  }
+  if (lane < k) ws->c[lane] = ws->s[lane] * acc;
+}
+
+// x += sum_j c_j V_j.
 template <typename TV, int KK, int W>
 __global__ void __launch_bounds__(kThreads) k_update_x(int64_t n, const TV* __restrict__ V, int64_t ldv,
                                                        Workspace* __restrict__ ws, double* __restrict__ x)
 {
-  __shared__ double coef[KK];
-  if (threadIdx.x == 0) {
-    double y[KK];
-#pragma unroll
-    for (int i = KK - 1; i >= 0; --i) {
-      double acc = ws->g[i];
-#pragma unroll
-      for (int j = i + 1; j < KK; ++j) acc -= ws->H[j][i] * y[j];
-      y[i] = acc / ws->H[i][i];
-    }
-#pragma unroll
-    for (int j = 0; j < KK; ++j) coef[j] = ws->s[j] * y[j];
-  }
   publish_pending(ws);
-  __syncthreads();
   double cj[KK];
 #pragma unroll
-  for (int j = 0; j < KK; ++j) cj[j] = coef[j];
+  for (int j = 0; j < KK; ++j) cj[j] = ws->c[j];
   const int64_t nv = n / W, stride = (int64_t)gridDim.x * kThreads;
   const int64_t t0 = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   for (int64_t i = t0; i < nv; i += stride) {
@@ -408,15 +474,12 @@ int step(int64_t n, int m, int k, TV* V, int64_t ldv, void* wsp, double* resid_o
     // pass B keeps every loaded value until the updated W is known: at most
     // two values per lane, so 32 stored vectors stay in registers
     constexpr int WB = W < 2 ? W : 2;
-    const int nb = grid_for(n, W);
     with_count<1>(k + 1, [&](auto KK_) {
       constexpr int KK = decltype(KK_)::value;
+      const int nb = grid_for(n, W, max_blocks(KK));
       hipLaunchKernelGGL((k_pass_a<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws);
-      hipLaunchKernelGGL((k_fin_a<KK>), dim3(1), dim3(kFinThreads), 0, st, nb, ws);
       hipLaunchKernelGGL((k_pass_b<TV, KK, WB>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws);
-      hipLaunchKernelGGL((k_fin_b<KK>), dim3(1), dim3(kFinThreads), 0, st, nb, ws);
-      hipLaunchKernelGGL((k_pass_c<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws);
-      hipLaunchKernelGGL((k_fin_c<KK>), dim3(1), dim3(kFinThreads), 0, st, nb, ws, resid_out);
+      hipLaunchKernelGGL((k_pass_c<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws, resid_out);
     });
   };
   if (packed<TV>(V, ldv)) launch(std::integral_constant<int, 4>{});
@@ -434,9 +497,10 @@ int update(int64_t n, int m, int k, const TV* V, int64_t ldv, void* wsp, double*
   Workspace* ws = static_cast<Workspace*>(wsp);
   auto launch = [&](auto W_) {
     constexpr int W = decltype(W_)::value;
+    hipLaunchKernelGGL(k_solve_cycle, dim3(1), dim3(64), 0, st, k, ws);
     with_count<1>(k, [&](auto KK_) {
       constexpr int KK = decltype(KK_)::value;
-      hipLaunchKernelGGL((k_update_x<TV, KK, W>), dim3(grid_for(n, W)), dim3(kThreads), 0, st, n, V, ldv, ws, x);
+      hipLaunchKernelGGL((k_update_x<TV, KK, W>), dim3(grid_for(n, W, 2 * kMaxBlocks)), dim3(kThreads), 0, st, n, V, ldv, ws, x);
     });
   };
   if (packed<TV>(V, ldv, x)) launch(std::integral_constant<int, 4>{});
