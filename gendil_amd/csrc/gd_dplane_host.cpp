@@ -28,6 +28,14 @@ int apply_diffusion(const gd_plan* plan, const T* x, T* y, hipStream_t s)
   if (plan->dim != 3 || plan->E >= (int64_t)1 << 31) return GD_ERR_UNSUPPORTED;
   const DEntry* en = find_diff(plan->desc.order + 1, plan->desc.num_quad);
   if (!en) return GD_ERR_UNSUPPORTED;
+  // Small meshes in FP64 leave this kernel a few blocks whose phases nothing
+  // hides: there the generic kernel is faster with q >= 4 where mu has
+  // several terms or n = 4 (9 x 8 x 10, generic against this: n = 4, q = 4 13.2 and 17.6 us, q = 6
+  // 12.6 and 20.9; n = 3, q = 4 14.4 and 15.6), and slower from 15 x 14 x 16 on
+  // (18.2 and 14.4; 26.8 and 18.6; 17.3 and 12.4).  q = 3, one term with n < 4
+  // and FP32 gain at every size measured.
+  if (sizeof(T) == 8 && en->Q >= 4 && plan->E < 2500 && (en->N == 4 || plan->term_rank[kTermMu] > 1))
+    return GD_ERR_UNSUPPORTED;
   const TableSet* ts = find_tables(plan, en->N, en->Q);
   DArgs<T> a;
   a.E = (int)plan->E;
