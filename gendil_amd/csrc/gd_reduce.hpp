@@ -1,7 +1,8 @@
 // Deterministic two-stage reductions shared by the Krylov kernels: every
 // block of a pass stores its column sums as partials (column-major, one
 // contiguous column per reduced quantity), and a one-block finishing kernel
-// sums them in a fixed order.  The kernel boundary between the two orders the
+// (CG, BiCGSTAB; the Arnoldi passes do it at the start of the next pass) sums
+// them in a fixed order.  The kernel boundary between the two orders the
 // partials; a device-scope fence in every block, the alternative, measured far
 // slower on the eight-XCD part.
 #pragma once
