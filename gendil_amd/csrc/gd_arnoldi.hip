@@ -31,9 +31,11 @@
 // (the next step's pass A or the cycle's update): a store to host memory at the
 // end of a kernel holds the kernel's completion for the bus round trip.
 //
-// FP32 bases are read 16 bytes per lane (4 values) where the basis and its
-// leading dimension are 16-byte aligned (pass B, which keeps every loaded
-// value live, 8 bytes); FP64 bases one value per lane, which measured as fast.
+// Bases are read 16 bytes per lane where the basis and its leading dimension
+// are 16-byte aligned (pass B in FP32, which keeps every loaded value live, 8
+// bytes): one block per CU needs that many bytes in flight (FP64 32^3, p = 3 with
+// 8 bytes per lane 315 ms a solve, with 16 300; 296 with the finishing kernels,
+// which smaller systems beat: 16^3 81.3 -> 64.1, 28^3 p = 2 42.8 -> 37.5).
 //
 // The cycle end solves the triangular system H y = g in one wave (with the last
 // column's finish) and adds x += sum_j s_j y_j V_j in FP64.
@@ -453,14 +455,14 @@ void with_count(int k, F&& f)
   }
 }
 
-// values per lane and access: 4 for a 16-byte aligned FP32 basis whose
-// leading dimension is a whole number of 16-byte packs (and 16-byte aligned x
-// for the update), else 1
+// 16-byte accesses: a 16-byte aligned basis (and x for the update) whose
+// leading dimension is a whole number of packs; else one value per lane
+template <typename TV>
+constexpr int kPack = 16 / (int)sizeof(TV);
 template <typename TV>
 bool packed(const void* V, int64_t ldv, const void* x = nullptr)
 {
-  return sizeof(TV) == 4 && reinterpret_cast<uintptr_t>(V) % 16 == 0 && (ldv * (int64_t)sizeof(TV)) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  return reinterpret_cast<uintptr_t>(V) % 16 == 0 && ldv % kPack<TV> == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 
 template <typename TV>
@@ -482,7 +484,7 @@ int step(int64_t n, int m, int k, TV* V, int64_t ldv, void* wsp, double* resid_o
       hipLaunchKernelGGL((k_pass_c<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws, resid_out);
     });
   };
-  if (packed<TV>(V, ldv)) launch(std::integral_constant<int, 4>{});
+  if (packed<TV>(V, ldv)) launch(std::integral_constant<int, kPack<TV>>{});
   else launch(std::integral_constant<int, 1>{});
   GD_HIP(hipGetLastError());
   return GD_OK;
@@ -503,7 +505,7 @@ int update(int64_t n, int m, int k, const TV* V, int64_t ldv, void* wsp, double*
       hipLaunchKernelGGL((k_update_x<TV, KK, W>), dim3(grid_for(n, W, 2 * kMaxBlocks)), dim3(kThreads), 0, st, n, V, ldv, ws, x);
     });
   };
-  if (packed<TV>(V, ldv, x)) launch(std::integral_constant<int, 4>{});
+  if (packed<TV>(V, ldv, x)) launch(std::integral_constant<int, kPack<TV>>{});
   else launch(std::integral_constant<int, 1>{});
   GD_HIP(hipGetLastError());
   return GD_OK;

@@ -303,8 +303,8 @@ int gd_add_f32_to_f64(int64_t n, double scale, const float* x, double* y, gd_str
  *     estimate) is stored there with a system-scope store (pinned host memory
  *     from gd_host_alloc is allowed and may be polled) by the first block of
  *     the next step or update on this workspace, early in that kernel, so no
- *     kernel's completion waits for the host write.  A 16-byte aligned FP32
- *     V with ldv a multiple of 4 runs 16-byte accesses.
+ *     kernel's completion waits for the host write.  A 16-byte aligned V
+ *     with rows of whole 16-byte packs runs 16-byte accesses.
  *   gd_gmres_update: x += V_{0..k-1} y with y from the k x k triangular
  *     system (gmres.hpp:240-265); stores the last step's residual estimate. */
 size_t gd_gmres_workspace_bytes(void);
