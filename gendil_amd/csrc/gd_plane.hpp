@@ -881,7 +881,8 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
       T b[Q][Q], u[N][N], A[N][N];
       beta_at(2, e, sub, sm, Q + s, T(1), b);
       const bool bnd = neighbour(e, sub, 2, s) < 0;
-      const T c = bnd && a.bc_none ? T(0) : a.adv_coef * a.detJ * a.invh[2];
+      const bool skip = bnd && a.bc_none;  // no flux, whatever the field is there (it may be infinite)
+      const T c = a.adv_coef * a.detJ * a.invh[2];
 #pragma unroll
       for (int m = 0; m < N; ++m)
 #pragma unroll
@@ -898,8 +899,9 @@ __global__ void __launch_bounds__((Geo<N, Q, ADV>::NT)) __attribute__((amdgpu_wa
 #pragma unroll
         for (int j = 0; j < Q; ++j) {
           const T dot = s ? b[k][j] : -b[k][j];
-          f[j] = c * (dot > T(0) ? dot * own[j] : dot * ext[j]);
-          if constexpr (FIELD == kPointwise) f[j] *= w[k] * w[j];
+          T up = c * (dot > T(0) ? dot * own[j] : dot * ext[j]);
+          if constexpr (FIELD == kPointwise) up *= w[k] * w[j];
+          f[j] = skip ? T(0) : up;
         }
         P::down(B, f, g);
 #pragma unroll

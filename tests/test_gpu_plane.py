@@ -179,3 +179,46 @@ def test_pointwise_transpose_with_mass():
     z = op.transpose(torch.as_tensor(r, device="cuda"), torch.empty(op.num_dofs, dtype=torch.float64, device="cuda"))
     P = oracle.Problem(fes, ir, mass_coef=0.6, adv_coef=-0.3, sigma=sigma, adv=(cell, faces))
     assert rel_l2(z.cpu().numpy(), P.apply_transpose(r)) <= 1e-12
+
+
+def pole(s):
+    with np.errstate(divide="ignore"):
+        return 1.0 / (s * (1.0 - s))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("basis", ["L", "G"])
+@pytest.mark.parametrize("mc", [0.0, 0.7])
+def test_field_infinite_on_skipped_boundary_faces(mc, basis, dtype):
+    """Without boundary data a boundary face carries no flux, whatever the field is there: a component with a pole on
+    its own axis's ends leaves a finite result."""
+    fe = G.MakeLobattoFiniteElement(2) if basis == "L" else G.MakeLegendreFiniteElement(2)
+    fes = G.MakeFiniteElementSpace(G.CartesianMesh([4, 2, 4], [0.25, 0.5, 0.25], [0.0] * 3, False), fe)
+    beta = VectorField([SeparableField([(0.1 * (d + 1), {d: pole})]) for d in range(3)])
+    check(fes, 4, dtype, beta, "none", None, mc, 1.0)
+
+
+def test_pointwise_field_unset_on_skipped_boundary_faces():
+    """The boundary rows of a per-point field are not used without boundary data: NaN there reaches neither the apply nor
+    the transpose, and the gradient is 0 there."""
+    sizes, n, q = (3, 4, 5), 3, 4
+    fes, ir = space(sizes, n - 1, "L", False), G.MakeIntegrationRule(q)
+    cell, faces, _ = pointwise_problem(fes, q, 3)
+    edge = []
+    for a in range(3):
+        ext = [s + (d == a) for d, s in enumerate(sizes)]
+        at = np.indices(ext[::-1]).reshape(3, -1)[2 - a]
+        edge.append((at == 0) | (at == sizes[a]))
+        faces[a][edge[a]] = np.nan
+    dev = [torch.as_tensor(t, device="cuda") for t in (cell, *faces)]
+    op = G.MakeAdvectionOperator(fes, ir, G.PointwiseField(dev[0], dev[1:]))
+    u, r = G.fill_random(op.num_dofs, 21), G.fill_random(op.num_dofs, 22)
+    P = oracle.Problem(fes, ir, adv_coef=1.0, adv=(cell, faces))
+    du, dr = torch.as_tensor(u, device="cuda"), torch.as_tensor(r, device="cuda")
+    assert rel_l2(op(du, torch.empty_like(du)).cpu().numpy(), P.apply(u)) <= 1e-12
+    assert rel_l2(op.transpose(dr, torch.empty_like(dr)).cpu().numpy(), P.apply_transpose(r)) <= 1e-12
+    dcell, dfaces = torch.empty_like(dev[0]), [torch.empty_like(t) for t in dev[1:]]
+    op.plan.grad_beta(1.0, du, dr, dcell, dfaces)
+    for a in range(3):
+        g = dfaces[a].cpu().numpy()
+        assert np.all(g[edge[a]] == 0.0) and np.all(np.isfinite(g))
