@@ -184,12 +184,19 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
   }
   __syncthreads();
 
+  // the field on a face as its flux takes it: outflow only at the boundary (none
+  // at all without data), where nothing else enters
+  auto face_beta = [&](double beta, bool upper, bool bnd) {
+    const double out = a.bc_none ? 0.0 : (upper ? fmax(beta, 0.0) : fmin(beta, 0.0));
+    return bnd ? out : beta;
+  };
   // the flux of one face point that this side's test function collects:
   // outflow c dot (own - nb), as the neighbour tests its inflow with -dot
+  // (unless dot < 0: what is not a number stays so)
   auto flux = [&](double c, double beta, bool upper, bool bnd, double own, double nb) {
     const double dot = upper ? beta : -beta;
     const double v = bnd ? own : own - nb;
-    return dot > 0.0 && !(bnd && a.bc_none) ? c * dot * v : 0.0;
+    return dot < 0.0 ? 0.0 : c * dot * v;
   };
 
   // ---- phase 2 ----
@@ -216,13 +223,13 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const double* src = a.beta_face[0] + face_index(a, sub, 0, s) * QQ + kz * Q;
+        xb[s] = mesh.neighbour(e, sub, 0, s) < 0;
 #pragma unroll
-        for (int k = 0; k < Q; ++k) fx[s][k] = src[k];
+        for (int k = 0; k < Q; ++k) fx[s][k] = face_beta(src[k], s, xb[s]);
         double nd[N];
 #pragma unroll
         for (int m = 0; m < N; ++m) nd[m] = r[2 * NN + s * N + m];
         P::up(B, nd, xn[s]);
-        xb[s] = mesh.neighbour(e, sub, 0, s) < 0;
       }
 #pragma unroll
       for (int k = 0; k < Q; ++k) {
@@ -267,9 +274,10 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
       for (int s = 0; s < 2; ++s) {  // y faces
         const double* src = a.beta_face[1] + face_index(a, sub, 1, s) * QQ + kz * Q;
+        const bool bnd = mesh.neighbour(e, sub, 1, s) < 0;
         double be[Q], nd[N], own[Q], ext[Q], f[Q], o[N];
 #pragma unroll
-        for (int k = 0; k < Q; ++k) be[k] = src[k];
+        for (int k = 0; k < Q; ++k) be[k] = face_beta(src[k], s, bnd);
         pin(A);
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -284,7 +292,6 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
         for (int i = 0; i < N; ++i) nd[i] = r[2 * NN + (2 + s) * N + i];
         P::up(B, nd, ext);
-        const bool bnd = mesh.neighbour(e, sub, 1, s) < 0;
 #pragma unroll
         for (int j = 0; j < Q; ++j) f[j] = flux(a.c[1] * wz * w[j], be[j], s, bnd, own[j], ext[j]);
         P::down(B, f, o);
@@ -345,7 +352,7 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
       for (int k = 0; k < Q; ++k) {
         double be[Q], t0[N], f[Q], o[N];
 #pragma unroll
-        for (int j = 0; j < Q; ++j) be[j] = src[k * Q + j];
+        for (int j = 0; j < Q; ++j) be[j] = face_beta(src[k * Q + j], s, bnd);
         pin(A);
         pin(u);
         P::row(B, u, k, t0);

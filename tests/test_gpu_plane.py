@@ -222,3 +222,20 @@ def test_pointwise_field_unset_on_skipped_boundary_faces():
     for a in range(3):
         g = dfaces[a].cpu().numpy()
         assert np.all(g[edge[a]] == 0.0) and np.all(np.isfinite(g))
+
+
+def test_nan_in_a_pointwise_face_field_reaches_the_transpose():
+    """NaN at a point of one inner face per axis: NaN in both elements of the face, nowhere else."""
+    sizes, n, q = (5, 3, 4), 3, 4
+    fes, ir = space(sizes, n - 1, "G", True), G.MakeIntegrationRule(q)
+    for a in range(3):
+        cell, faces, _ = pointwise_problem(fes, q, 4)
+        faces[a][2 + 5 * 2 + 15 * 2, 7] = np.nan
+        dev = [torch.as_tensor(t, device="cuda") for t in (cell, *faces)]
+        op = G.MakeAdvectionOperator(fes, ir, G.PointwiseField(dev[0], dev[1:]))
+        r = G.fill_random(op.num_dofs, 22)
+        dr = torch.as_tensor(r, device="cuda")
+        got = op.transpose(dr, torch.empty_like(dr)).cpu().numpy()
+        want = oracle.Problem(fes, ir, adv_coef=1.0, adv=(cell, faces)).apply_transpose(r)
+        assert np.isnan(want).sum() == 2 * n**3
+        assert np.array_equal(np.isnan(got), np.isnan(want))
