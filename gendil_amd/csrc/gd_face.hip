@@ -629,14 +629,39 @@ int check_plan(const gd_plan* pl, const char* what)
   return GD_OK;
 }
 
+// true when [a, a + na) and [b, b + nb) share storage
+bool overlap(const double* a, int64_t na, const double* b, int64_t nb)
+{
+  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+  return a0 < b0 + (uintptr_t)nb * sizeof(double) && b0 < a0 + (uintptr_t)na * sizeof(double);
+}
+
+// whether the two sides of an interface may add to the same element: their
+// parts of y share storage and are not different layers of one space (a mesh
+// one cell thick, glued to itself, has the same element on both sides)
+bool sides_share_elements(const Args& a)
+{
+  const Side &m = a.s[0], &p = a.s[1];
+  auto size = [&](const Side& s) {
+    int64_t n = 1;
+    for (int d = 0; d < a.D; ++d) n *= s.M[d] * s.n;
+    return n;
+  };
+  if (!overlap(m.y, size(m), p.y, size(p))) return false;
+  const bool one_space = m.y == p.y && m.n == p.n && std::equal(m.M, m.M + a.D, p.M);
+  return !one_space || m.base == p.base;
+}
+
 int launch(const Args& args, hipStream_t st)
 {
   if (args.nfaces <= 0) return GD_OK;
   // conforming 3D interfaces of the common orders and rules: one wave per few
-  // faces.  (Interior faces by colour and subfaces keep the kernel below.)
+  // faces.  (Interior faces by colour and subfaces keep the kernel below, and
+  // so do sides that may share elements: this kernel adds both at once, that
+  // one after the other.)
   if (args.D == 3 && args.s[0].stride == 0 && args.s[1].stride == 0 && !args.s[0].Bmap && !args.s[1].Bmap &&
       args.wscale == 1.0 && std::max({args.s[0].n, args.s[1].n, args.q}) <= kWaveN &&
-      args.nfaces < (1LL << 31) - 64) {
+      args.nfaces < (1LL << 31) - 64 && !sides_share_elements(args)) {
     Args a = args;
     a.fpb = std::max(1, 64 / (a.q * a.q));
     const long long blocks = (a.nfaces + a.fpb - 1) / a.fpb;
@@ -690,13 +715,6 @@ int common_args(const gd_plan* m, const gd_plan* p, int axis, int sign, Args& a,
   if (!ts) return fail(GD_ERR_UNSUPPORTED, "face operator: plan has no tables for its rule");
   a.geo = make_params<double>(m, ts, 0.0, 1.0);
   return GD_OK;
-}
-
-// true when [a, a + na) and [b, b + nb) share storage
-bool overlap(const double* a, int64_t na, const double* b, int64_t nb)
-{
-  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
-  return a0 < b0 + (uintptr_t)nb * sizeof(double) && b0 < a0 + (uintptr_t)na * sizeof(double);
 }
 
 // x is read while y is added into (in several launches for the coloured and

@@ -52,3 +52,23 @@ def test_range_of_orders_and_rules(bases, n, q):
 @pytest.mark.parametrize("sizes", [(1, 1, 1), (9, 2, 7), (1, 1, 65)], ids=str)
 def test_face_counts(sizes):
     check(1, list(sizes), (3, 2), "LL", 3, "c2")
+
+
+@pytest.mark.parametrize("thick", [1, 2])
+@pytest.mark.parametrize("basis,n", [("L", 1), ("G", 2), ("L", 3), ("G", 4)])
+@pytest.mark.parametrize("face", [0, 2, 4])
+def test_space_glued_to_itself(face, basis, n, thick):
+    """One space on both sides, closing the face's axis: with one cell along it both sides are the same element, whose
+    values both shares are added to."""
+    sizes, h, origin, q = [5, 4, 7], [0.3, 0.2, 0.25], [0.1, -0.2, 0.3], max(n, 2)
+    sizes[face % 3] = thick
+    make = G.MakeLobattoFiniteElement if basis == "L" else G.MakeLegendreFiniteElement
+    fes = G.MakeFiniteElementSpace(G.CartesianMesh(sizes, h, origin), make(n - 1))
+    op = G.MakeAdvectionFaceOperator(fes, fes, G.CartesianIntermeshFaceConnectivity(3, face, sizes, sizes),
+                                     G.MakeIntegrationRule(q), beta_field("trig", 3))
+    x, y0 = G.fill_random(fes.num_dofs, 3), G.fill_random(fes.num_dofs, 4)
+    y = op(torch.as_tensor(x, device="cuda"), torch.as_tensor(y0, device="cuda"))
+    side = dict(sizes=sizes, h=h, origin=origin, n=n, basis="LG".index(basis))
+    want = y0.copy()
+    oracle.intermesh_operator(face, q, side, side, beta_numpy("trig", 3), x, x, want, want)
+    assert rel_l2(y.cpu().numpy() - y0, want - y0) <= 1e-12
