@@ -88,6 +88,22 @@ int k3_choice(const gd_plan* plan, int N, bool adv, bool mass)
   return 1;
 }
 
+// 4D-6D: the kernel of a forward apply, 0 for the generic one.  What is pinned
+// where it serves; else, unless the generic kernel is pinned, the two-node
+// Kronecker kernel (order 1, constant coefficients: GenDiL's 6D benchmark
+// operator, 5^6 elements: see n2k), then the Kronecker kernel (the 6D p = 2
+// q = 3 phase-space apply of 19.7 M unknowns takes 163 us there and 2,650 us on
+// the generic kernel).
+template <typename T>
+int highdim_choice(const gd_plan* plan, bool adv, bool mass)
+{
+  const int tuned = tuned_lanes(plan, 0, sizeof(T));
+  if (tuned == 0) return 0;
+  if (tuned == kron::kVariant && kron::available(plan, adv, mass)) return kron::kVariant;
+  if (n2k::available<T>(plan, adv, mass)) return n2k::kVariant;
+  return kron::preferred(plan, adv, mass) ? kron::kVariant : 0;
+}
+
 // The register-resident kernel covers 3D GLL elements with q = p+1 and
 // one-axis separable (or constant) coefficients; see gd_k3d_host.cpp.
 template <typename T>
@@ -130,21 +146,12 @@ int apply_impl(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, h
     if (adv && plan->beta_kind == GD_BETA_POINTWISE)
       return fail(GD_ERR_UNSUPPORTED, "pointwise beta is FP64 only");
   }
-  // 4D-6D, order 1, constant coefficients: the two-node Kronecker kernel
-  // unless the generic kernel (0) is pinned (measured on MI355X for GenDiL's
-  // 6D benchmark operator, 5^6 elements: see n2k)
-  if (plan->dim >= 4 && tuned_lanes(plan, 2, sizeof(T)) != 0 && n2k::available<T>(plan, adv, mass_coef != T(0))) {
-    const int r = n2k::apply<T>(plan, mass_coef, adv_coef, x, y, s);
-    if (r != GD_ERR_UNSUPPORTED) return r;
-  }
-  // 4D-6D sums of Kronecker products: the 6D p = 2 q = 3 phase-space apply of
-  // 19.7 M unknowns takes 163 us here and 2,650 us on the generic kernel
   if (plan->dim >= 4) {
-    const int tuned = tuned_lanes(plan, 0, sizeof(T));
-    if (tuned == kron::kVariant || (tuned != 0 && kron::preferred(plan, adv, mass_coef != T(0)))) {
-      const int r = kron::apply<T>(plan, mass_coef, adv_coef, x, y, s);
-      if (r != GD_ERR_UNSUPPORTED) return r;
-    }
+    const int kind = highdim_choice<T>(plan, adv, mass_coef != T(0));
+    int r = GD_ERR_UNSUPPORTED;
+    if (kind == n2k::kVariant) r = n2k::apply<T>(plan, mass_coef, adv_coef, x, y, s);
+    if (kind == kron::kVariant) r = kron::apply<T>(plan, mass_coef, adv_coef, x, y, s);
+    if (r != GD_ERR_UNSUPPORTED) return r;
   }
   if (tuned_lanes(plan, 0, sizeof(T)) == pl::kVariant) {
     const int r = pl::apply<T>(plan, mass_coef, adv_coef, x, y, s);
@@ -322,14 +329,9 @@ int gd_plan_query_variant(const gd_plan* plan, int32_t precision_bytes, double m
   const int N = plan->desc.order + 1;
   auto resolve = [&](auto tag) -> int {
     using T = decltype(tag);
-    if (plan->dim >= 4 && plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1] != 0 &&
-        gd::n2k::available<T>(plan, adv, mass))
-      return gd::n2k::kVariant;
     if (plan->dim >= 4) {
-      const int tuned = plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1];
-      if (tuned == gd::kron::kVariant ? gd::kron::available(plan, adv, mass)
-                                      : tuned != 0 && gd::kron::preferred(plan, adv, mass))
-        return gd::kron::kVariant;
+      const int kind = gd::highdim_choice<T>(plan, adv, mass);
+      if (kind != 0) return kind;
     }
     if (plan->tuned_k3_lanes[sizeof(T) == 8 ? 0 : 1] == gd::pl::kVariant && gd::pl::available<T>(plan, adv, mass))
       return gd::pl::kVariant;

@@ -97,3 +97,15 @@ def test_what_it_refuses_and_where_it_is_the_default():
     op = G.MakeAdvectionOperator(fes, ir, mixed_field(4))
     op.plan.set_variant(torch.float64, 0)
     assert op.plan.query_variant(torch.float64, 0.0, 1.0) == 0
+
+
+def test_pinned_where_the_two_node_kernel_also_serves():
+    """Order 1 with constant coefficients: the two-node kernel by default, the Kronecker kernel once pinned."""
+    beta = VectorField([SeparableField.constant(c) for c in (1.0, -0.5, 0.25, 2.0)])
+    run(4, 2, 2, "L", [5, 3, 2, 3], False, beta, 0.0, None, 0.6, 0.3)
+    mesh = G.CartesianMesh([5, 3, 2, 3], [0.2] * 4, [0.0] * 4, False)
+    op = G.MakeAdvectionOperator(G.MakeFiniteElementSpace(mesh, G.MakeLobattoFiniteElement(1)), G.MakeIntegrationRule(2), beta)
+    assert op.plan.query_variant(torch.float64, 0.0, 1.0) == 64
+    for variant in (KRON, 64):
+        op.plan.set_variant(torch.float64, variant)
+        assert op.plan.query_variant(torch.float64, 0.0, 1.0) == variant
