@@ -311,6 +311,7 @@ int gd_plan_autotune(gd_plan* plan, int32_t precision_bytes, double mass_coef, d
     return rc;
   }
   *knob = best_lanes;
+  plan->generic_pinned[slot] = false;
   if (chosen) *chosen = best_lanes;
   if (best_ms) *best_ms = best;
   return GD_OK;
@@ -361,6 +362,7 @@ int gd_plan_set_variant(gd_plan* plan, int32_t precision_bytes, int32_t lanes)
       lanes != gd::kron::kVariant)
     return fail(GD_ERR_INVALID, "gd_plan_set_variant: bad arguments");
   plan->tuned_k3_lanes[slot] = lanes;
+  plan->generic_pinned[slot] = lanes == 0;
   return GD_OK;
 }
 

@@ -25,6 +25,7 @@ const DEntry* find_diff(int N, int Q)
 template <typename T>
 int apply_diffusion(const gd_plan* plan, const T* x, T* y, hipStream_t s)
 {
+  if (plan->generic_pinned[sizeof(T) == 8 ? 0 : 1]) return GD_ERR_UNSUPPORTED;
   if (plan->dim != 3 || plan->E >= (int64_t)1 << 31) return GD_ERR_UNSUPPORTED;
   const DEntry* en = find_diff(plan->desc.order + 1, plan->desc.num_quad);
   if (!en) return GD_ERR_UNSUPPORTED;

@@ -182,6 +182,10 @@ struct gd_plan {
   // 0 = generic kernel, 1/2/4 = register kernel with that many lanes per
   // element, 16 + lanes = Kronecker-factored kernel
   int tuned_k3_lanes[2] = {-1, -1};
+  // variant 0 pinned by gd_plan_set_variant (not chosen by the autotuner, which
+  // times forward applies alone): transpose, field gradient and 3D diffusion
+  // stay on their generic kernels too
+  bool generic_pinned[2] = {false, false};
   // p-adaptive path: kernel variant per precision (-1 = default), lazily
   // built element buckets and device parameter block, and a counter bumped by
   // every coefficient change so the device copy is refreshed

@@ -11,6 +11,7 @@ namespace {
 
 const AdjEntry* serving(const gd_plan* plan)
 {
+  if (plan->generic_pinned[0]) return nullptr;
   if (plan->dim != 3 || plan->padapt || plan->E >= (int64_t)1 << 31 || plan->beta_kind != GD_BETA_POINTWISE)
     return nullptr;
   const int N = plan->desc.order + 1, Q = plan->desc.num_quad;

@@ -182,7 +182,7 @@ class Plan:
         return chosen.value, best.value
 
     def set_variant(self, dtype, lanes: int):
-        """Pin the kernel variant: -1 default, 0 generic, 1/2/4 lanes per element
+        """Pin the kernel variant: -1 default, 0 generic (transpose, field gradient and diffusion too), 1/2/4 lanes per element
         (register kernel), 17/18/20 (Kronecker kernel, 16 + lanes), 48..55 (LDS-staged
         Kronecker kernel: +1 outputs staged through LDS, +2 128-thread blocks, +4 one term at
         a time), 56 / 57 (streaming form: one wave per block, persistent; 56 one tile buffer and two

@@ -235,7 +235,9 @@ int gd_plan_autotune(gd_plan* plan, int32_t precision_bytes, double mass_coef, d
  * Kronecker kernel, 4D-6D), 72 (plane kernel, 3D),
  * 73 (Kronecker kernel, 4D-6D); p-adaptive plans the variant index as reported by
  * gd_plan_autotune.  A pinned variant that does not serve a later apply
- * falls back to the default for that apply. */
+ * falls back to the default for that apply.  A pinned 0 also keeps the
+ * transpose, the field gradient and the 3D diffusion apply of that precision
+ * on their generic kernels. */
 int gd_plan_set_variant(gd_plan* plan, int32_t precision_bytes, int32_t lanes);
 /* The variant an apply with these coefficients would run now (after falling
  * back from a pinned variant that does not serve the plan), in the codes above. */

@@ -239,3 +239,41 @@ def test_nan_in_a_pointwise_face_field_reaches_the_transpose():
         want = oracle.Problem(fes, ir, adv_coef=1.0, adv=(cell, faces)).apply_transpose(r)
         assert np.isnan(want).sum() == 2 * n**3
         assert np.array_equal(np.isnan(got), np.isnan(want))
+
+
+def pinned(op, dtype, run):
+    """run() by default and with the generic kernel pinned: other sums, so other last bits."""
+    default = run()
+    op.plan.set_variant(dtype, 0)
+    generic = run()
+    op.plan.set_variant(dtype, -1)
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    for a, b in zip(default, generic):
+        assert not torch.equal(a, b) and rel_l2(a.double().cpu().numpy(), b.double().cpu().numpy()) <= tol
+    assert all(torch.equal(a, b) for a, b in zip(default, run()))
+
+
+@pytest.mark.parametrize("bc", ["none", "poly"])
+@pytest.mark.parametrize("basis", ["L", "G"])
+@pytest.mark.parametrize("n,q", PAIRS)
+def test_pinned_generic_kernels_of_the_pointwise_field(n, q, basis, bc):
+    fes = space((4, 5, 3), n - 1, basis, [False, True, False])
+    _, _, dev = pointwise_problem(fes, q, 7)
+    op = G.MakeAdvectionOperator(fes, G.MakeIntegrationRule(q), G.PointwiseField(dev[0], dev[1:]), bc_field(bc, 3))
+    u, r = (torch.as_tensor(G.fill_random(op.num_dofs, s), device="cuda") for s in (21, 22))
+
+    def run():
+        dcell, dfaces = torch.empty_like(dev[0]), [torch.empty_like(t) for t in dev[1:]]
+        op.plan.grad_beta(0.7, u, r, dcell, dfaces)
+        return [op.transpose(r, torch.empty_like(r)), dcell, *dfaces]
+
+    pinned(op, torch.float64, run)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("n,q", DIFF_PAIRS)
+def test_pinned_generic_kernel_of_the_diffusion(n, q, dtype):
+    fes = space((17, 13, 12), n - 1, "G", [True, False, True])
+    op = G.MakeDiffusionOperator(fes, G.MakeIntegrationRule(q), diffusivity_field("trig", 3), -1.0, 9.0)
+    x = torch.as_tensor(G.fill_random(op.num_dofs, 13), dtype=dtype, device="cuda")
+    pinned(op, dtype, lambda: [op(x, torch.empty_like(x))])
