@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <set>
 #include <string>
 #include <utility>
@@ -245,58 +246,76 @@ void free_fields(gd_plan* p)
   for (void* t : p->field_tables) (void)hipFree(t);
   p->field_tables.clear();
   if (p->fields64) (void)hipFree(p->fields64);
-  if (p->fields32) (void)hipFree(p->fields32);
-  p->fields64 = p->fields32 = nullptr;
+  p->fields64 = p->fields32 = nullptr;  // one allocation
+  p->terms64 = nullptr;
+  p->terms32 = nullptr;
 }
 
-// One allocation and one copy: the field descriptors and, for 3D plans, the
-// terms list built from them (fields f: [0..3) beta, 3 sigma, 4 bc, 5 mu).
+// The field descriptors of one precision and, for 3D plans, the terms list
+// built from them (fields f: [0..3) beta, 3 sigma, 4 bc, 5 mu), written to
+// `host`, the host image of device memory at `dev`.
 template <typename T>
-int upload_descriptors(gd_plan* p, const std::vector<FieldDev<T>>& f, void** dst, const FieldTerms<T>** terms)
+struct Descriptors {
+  FieldDev<T> fields[kMaxDim + 3];
+  FieldTerms<T> terms;
+};
+
+template <typename T>
+void put_descriptors(gd_plan* p, const std::vector<FieldDev<T>>& f, const Descriptors<T>* dev, Descriptors<T>& host)
 {
-  const size_t head = f.size() * sizeof(FieldDev<T>);
-  std::vector<char> blob(head + (p->dim == 3 ? sizeof(FieldTerms<T>) : 0));
-  std::memcpy(blob.data(), f.data(), head);
-  GD_HIP(hipMalloc(dst, blob.size()));
-  if (p->dim == 3) {
-    static const int from[kTermFields] = {3, 0, 1, 2, 4, 5};  // sigma, beta, bc, mu
-    FieldTerms<T> t;
-    std::memset(&t, 0, sizeof(t));
-    int n = 0;
-    for (int i = 0; i < kTermFields; ++i) {
-      const FieldDev<T>& src = f[from[i]];
-      t.first[i] = n;
-      t.rank[i] = src.rank;
-      for (int r = 0; r < src.rank; ++r) {
-        T scale = src.scale[r];
-        int bits = 0;
-        for (int d = 0; d < 3; ++d)
-          if (src.tab[r][d]) {
-            bits |= 1 << d;
-            t.axis[n] = d;
-            t.scale[n] = scale;
-            t.tab[n++] = src.tab[r][d];
-            scale = T(1);
-          }
-        if (!bits) {
-          bits = 4;
-          t.axis[n] = kRowConstant;
+  std::copy(f.begin(), f.end(), host.fields);
+  if (p->dim != 3) return;
+  static const int from[kTermFields] = {3, 0, 1, 2, 4, 5};  // sigma, beta, bc, mu
+  FieldTerms<T>& t = host.terms;
+  int n = 0;
+  for (int i = 0; i < kTermFields; ++i) {
+    const FieldDev<T>& src = f[from[i]];
+    t.first[i] = n;
+    t.rank[i] = src.rank;
+    for (int r = 0; r < src.rank; ++r) {
+      T scale = src.scale[r];
+      int bits = 0;
+      for (int d = 0; d < 3; ++d)
+        if (src.tab[r][d]) {
+          bits |= 1 << d;
+          t.axis[n] = d;
           t.scale[n] = scale;
-          t.tab[n++] = static_cast<const T*>(*dst);  // this block: longer than the q + 2 samples of one element
+          t.tab[n++] = src.tab[r][d];
+          scale = T(1);
         }
-        t.mask[i] |= bits << (3 * r);
+      if (!bits) {
+        bits = 4;
+        t.axis[n] = kRowConstant;
+        t.scale[n] = scale;
+        t.tab[n++] = reinterpret_cast<const T*>(dev);  // this block: longer than the q + 2 samples of one element
       }
+      t.mask[i] |= bits << (3 * r);
     }
-    t.first[kTermFields] = n;
-    for (int i = 0; i <= kTermFields; ++i) p->term_first[i] = t.first[i];
-    for (int i = 0; i < kTermFields; ++i) {
-      p->term_rank[i] = t.rank[i];
-      p->term_mask[i] = t.mask[i];
-    }
-    std::memcpy(blob.data() + head, &t, sizeof(t));
   }
-  GD_HIP(hipMemcpy(*dst, blob.data(), blob.size(), hipMemcpyHostToDevice));
-  *terms = p->dim == 3 ? reinterpret_cast<const FieldTerms<T>*>(static_cast<char*>(*dst) + head) : nullptr;
+  t.first[kTermFields] = n;
+  for (int i = 0; i <= kTermFields; ++i) p->term_first[i] = t.first[i];
+  for (int i = 0; i < kTermFields; ++i) {
+    p->term_rank[i] = t.rank[i];
+    p->term_mask[i] = t.mask[i];
+  }
+}
+
+// Both precisions' descriptors in one allocation and one copy.
+int upload_descriptors(gd_plan* p, const std::vector<FieldDev<double>>& f64, const std::vector<FieldDev<float>>& f32)
+{
+  struct Both {
+    Descriptors<double> d;
+    Descriptors<float> f;
+  };
+  GD_HIP(hipMalloc(&p->fields64, sizeof(Both)));
+  const Both* dev = static_cast<const Both*>(p->fields64);
+  p->fields32 = const_cast<FieldDev<float>*>(dev->f.fields);
+  auto host = std::make_unique<Both>();  // zeros
+  put_descriptors(p, f64, &dev->d, host->d);
+  put_descriptors(p, f32, &dev->f, host->f);
+  GD_HIP(hipMemcpy(p->fields64, host.get(), sizeof(Both), hipMemcpyHostToDevice));
+  p->terms64 = p->dim == 3 ? &dev->d.terms : nullptr;
+  p->terms32 = p->dim == 3 ? &dev->f.terms : nullptr;
   return GD_OK;
 }
 
@@ -339,9 +358,7 @@ int upload_fields(gd_plan* p)
   }
   p->fields64_host = f64;
   p->fields32_host = f32;
-  if (int rc = upload_descriptors(p, f64, &p->fields64, &p->terms64)) return rc;
-  if (int rc = upload_descriptors(p, f32, &p->fields32, &p->terms32)) return rc;
-  return GD_OK;
+  return upload_descriptors(p, f64, f32);
 }
 
 // Every coefficient change ends here.  Applies queued earlier on any stream
