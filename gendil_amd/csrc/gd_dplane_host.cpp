@@ -53,7 +53,7 @@ int apply_diffusion(const gd_plan* plan, const T* x, T* y, hipStream_t s)
   a.gll = plan->desc.basis == GD_BASIS_GLL;
   const Tables1D<T>* tab;
   if constexpr (std::is_same_v<T, double>) {
-    tab = &ts->t64;
+    tab = &ts->once64;
     a.terms = plan->terms64;
   } else {
     tab = &ts->t32;

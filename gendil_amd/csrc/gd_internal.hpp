@@ -108,13 +108,26 @@ struct Params {
   int num_blocks;
 };
 
-struct TableSet {
+template <class R>
+struct RuleTables {
+  std::vector<R> B, Gq, b0, b1, w, xq, Gb, d0, d1;
+};
+
+// The tables as FP64 arithmetic gives them (a few units off in the last place),
+// and the same from extended precision.  Kernels that hold half of a table and
+// mirror it, or products of tables, read the latter, rounded once: there an
+// entry's error meets itself in every sum (n = 3..5 on Lobatto nodes, 3D apply:
+// up to 1.5 times the generic kernel's error against an extended-precision
+// apply with the former, at most 0.7 times with the latter).  The others keep
+// the former and with it their bits (iteration counts of a solve on a mass
+// operator are compared with GenDiL's).
+struct TableSet : RuleTables<double> {
   int n = 0, q = 0;
   void* dev64 = nullptr;  // contiguous device block (double)
   void* dev32 = nullptr;  // contiguous device block (float)
-  Tables1D<double> t64{};
+  Tables1D<double> t64{}, once64{};
   Tables1D<float> t32{};
-  std::vector<double> B, Gq, b0, b1, w, xq, Gb, d0, d1;  // host copies
+  RuleTables<long double> ext;
 };
 
 struct HostField {

@@ -47,7 +47,7 @@ AdjArgs pack(const gd_plan* plan, double mass_coef, double adv_coef)
   const FieldDev<double>* f = static_cast<const FieldDev<double>*>(plan->fields64);
   a.sigma = f + 3;
   a.bc = f + 4;
-  const Tables1D<double>& t = find_tables(plan, plan->desc.order + 1, plan->desc.num_quad)->t64;
+  const Tables1D<double>& t = find_tables(plan, plan->desc.order + 1, plan->desc.num_quad)->once64;
   a.B = t.B;
   a.Gb = t.Gb;
   a.b0 = t.b0;

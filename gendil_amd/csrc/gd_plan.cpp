@@ -44,40 +44,47 @@ int hip_fail(hipError_t e, const char* what)
 namespace {
 
 // returns P_n(t), P_{n-1}(t)
-std::pair<double, double> legendre_pair(int n, double t)
+template <class R>
+std::pair<R, R> legendre_pair(int n, R t)
 {
-  double pm1 = 1.0, p = t;
+  R pm1 = 1.0, p = t;
   if (n == 0) return {1.0, 0.0};
   for (int k = 1; k < n; ++k) {
-    const double pn = ((2 * k + 1) * t * p - k * pm1) / (k + 1);
+    const R pn = ((2 * k + 1) * t * p - k * pm1) / (k + 1);
     pm1 = p;
     p = pn;
   }
   return {p, pm1};
 }
 
-void rule_gl(int n, double* x, double* w)
+// the last Newton step's size, relative
+template <class R>
+constexpr R kStep = sizeof(R) > sizeof(double) ? R(1e-19L) : R(1e-16);
+
+template <class R>
+void rule_gl(int n, R* x, R* w)
 {
   for (int i = 0; i < (n + 1) / 2; ++i) {
-    double t = std::cos(M_PI * (i + 0.75) / (n + 0.5));  // descending roots
+    R t = std::cos(M_PI * (i + 0.75) / (n + 0.5));  // descending roots
     for (int it = 0; it < 64; ++it) {
       auto [p, pm1] = legendre_pair(n, t);
-      const double dp = n * (t * p - pm1) / (t * t - 1.0);
-      const double step = p / dp;
+      const R dp = n * (t * p - pm1) / (t * t - 1);
+      const R step = p / dp;
       t -= step;
-      if (std::fabs(step) <= 1e-16 * std::fabs(t) + 1e-300) break;
+      if (std::fabs(step) <= kStep<R> * std::fabs(t) + R(1e-300)) break;
     }
     auto [p, pm1] = legendre_pair(n, t);
-    const double dp = n * (t * p - pm1) / (t * t - 1.0);
-    const double wt = 1.0 / ((1.0 - t * t) * dp * dp);  // half of 2/((1-t^2)P'^2)
-    x[n - 1 - i] = 0.5 + 0.5 * t;
-    x[i] = 0.5 - 0.5 * t;
+    const R dp = n * (t * p - pm1) / (t * t - 1);
+    const R wt = 1 / ((1 - t * t) * dp * dp);  // half of 2/((1-t^2)P'^2)
+    x[n - 1 - i] = R(0.5) + R(0.5) * t;
+    x[i] = R(0.5) - R(0.5) * t;
     w[i] = w[n - 1 - i] = wt;
   }
   if (n % 2) x[n / 2] = 0.5;
 }
 
-void rule_gll(int n, double* x, double* w)
+template <class R>
+void rule_gll(int n, R* x, R* w)
 {
   if (n == 1) {  // single node at the centre (GLLpoints.hpp one-point rule)
     x[0] = 0.5;
@@ -86,31 +93,32 @@ void rule_gll(int n, double* x, double* w)
   }
   const int m = n - 1;
   for (int i = 0; i < (n + 1) / 2; ++i) {
-    double t = std::cos(M_PI * i / m);
+    R t = std::cos(M_PI * i / m);
     if (i > 0) {
       for (int it = 0; it < 64; ++it) {
         auto [p, pm1] = legendre_pair(m, t);
-        const double dp = m * (t * p - pm1) / (t * t - 1.0);
-        const double d2p = (2.0 * t * dp - m * (m + 1.0) * p) / (1.0 - t * t);
-        const double step = dp / d2p;
+        const R dp = m * (t * p - pm1) / (t * t - 1);
+        const R d2p = (2 * t * dp - m * (m + R(1)) * p) / (1 - t * t);
+        const R step = dp / d2p;
         t -= step;
-        if (std::fabs(step) <= 1e-16 * std::fabs(t) + 1e-300) break;
+        if (std::fabs(step) <= kStep<R> * std::fabs(t) + R(1e-300)) break;
       }
     }
     auto [p, pm1] = legendre_pair(m, t);
     (void)pm1;
-    const double wt = 1.0 / (m * (m + 1.0) * p * p);
-    x[n - 1 - i] = (i == 0) ? 1.0 : 0.5 + 0.5 * t;
-    x[i] = (i == 0) ? 0.0 : 0.5 - 0.5 * t;
+    const R wt = 1 / (m * (m + R(1)) * p * p);
+    x[n - 1 - i] = (i == 0) ? 1.0 : R(0.5) + R(0.5) * t;
+    x[i] = (i == 0) ? 0.0 : R(0.5) - R(0.5) * t;
     w[i] = w[n - 1 - i] = wt;
   }
   if (n % 2) x[n / 2] = 0.5;
 }
 
 // Lagrange basis through nodes xs (lagrangeshapefunctions.hpp:37-86 math).
-double lag(const std::vector<double>& xs, int k, double x)
+template <class R>
+R lag(const std::vector<R>& xs, int k, R x)
 {
-  double num = 1.0, den = 1.0;
+  R num = 1.0, den = 1.0;
   for (int i = 0; i < (int)xs.size(); ++i)
     if (i != k) {
       num *= x - xs[i];
@@ -119,12 +127,13 @@ double lag(const std::vector<double>& xs, int k, double x)
   return num / den;
 }
 
-double dlag(const std::vector<double>& xs, int k, double x)
+template <class R>
+R dlag(const std::vector<R>& xs, int k, R x)
 {
-  double s = 0.0;
+  R s = 0.0;
   for (int i = 0; i < (int)xs.size(); ++i) {
     if (i == k) continue;
-    double num = 1.0, den = xs[k] - xs[i];
+    R num = 1.0, den = xs[k] - xs[i];
     for (int j = 0; j < (int)xs.size(); ++j)
       if (j != i && j != k) {
         num *= x - xs[j];
@@ -135,11 +144,10 @@ double dlag(const std::vector<double>& xs, int k, double x)
   return s;
 }
 
-int build_tables(int basis, int n, int q, TableSet& ts)
+template <class R>
+void compute_tables(int basis, int n, int q, RuleTables<R>& ts)
 {
-  ts.n = n;
-  ts.q = q;
-  std::vector<double> xn(n), wn(n);
+  std::vector<R> xn(n), wn(n);
   if (basis == GD_BASIS_GLL) rule_gll(n, xn.data(), wn.data());
   else rule_gl(n, xn.data(), wn.data());
   ts.xq.resize(q);
@@ -154,8 +162,8 @@ int build_tables(int basis, int n, int q, TableSet& ts)
   for (int a = 0; a < q; ++a)
     for (int b = 0; b < q; ++b) ts.Gq[a * q + b] = dlag(ts.xq, b, ts.xq[a]);
   for (int i = 0; i < n; ++i) {
-    ts.b0[i] = lag(xn, i, 0.0);
-    ts.b1[i] = lag(xn, i, 1.0);
+    ts.b0[i] = lag(xn, i, R(0));
+    ts.b1[i] = lag(xn, i, R(1));
   }
   ts.Gb.resize((size_t)q * n);
   for (int a = 0; a < q; ++a)
@@ -163,21 +171,27 @@ int build_tables(int basis, int n, int q, TableSet& ts)
   ts.d0.resize(n);
   ts.d1.resize(n);
   for (int i = 0; i < n; ++i) {
-    ts.d0[i] = dlag(xn, i, 0.0);
-    ts.d1[i] = dlag(xn, i, 1.0);
+    ts.d0[i] = dlag(xn, i, R(0));
+    ts.d1[i] = dlag(xn, i, R(1));
   }
-  // device upload: B | Gq | b0 | b1 | w | xq | Gb | d0 | d1
+}
+
+int build_tables(int basis, int n, int q, TableSet& ts)
+{
+  ts.n = n;
+  ts.q = q;
+  compute_tables<double>(basis, n, q, ts);
+  compute_tables<long double>(basis, n, q, ts.ext);
+  // device upload: B | Gq | b0 | b1 | w | xq | Gb | d0 | d1, then (FP64) the same rounded once
   std::vector<double> blob;
-  blob.insert(blob.end(), ts.B.begin(), ts.B.end());
-  blob.insert(blob.end(), ts.Gq.begin(), ts.Gq.end());
-  blob.insert(blob.end(), ts.b0.begin(), ts.b0.end());
-  blob.insert(blob.end(), ts.b1.begin(), ts.b1.end());
-  blob.insert(blob.end(), ts.w.begin(), ts.w.end());
-  blob.insert(blob.end(), ts.xq.begin(), ts.xq.end());
-  blob.insert(blob.end(), ts.Gb.begin(), ts.Gb.end());
-  blob.insert(blob.end(), ts.d0.begin(), ts.d0.end());
-  blob.insert(blob.end(), ts.d1.begin(), ts.d1.end());
+  auto append = [&](const auto& t) {
+    for (const auto* v : {&t.B, &t.Gq, &t.b0, &t.b1, &t.w, &t.xq, &t.Gb, &t.d0, &t.d1})
+      blob.insert(blob.end(), v->begin(), v->end());
+  };
+  append(static_cast<const RuleTables<double>&>(ts));
+  const size_t len = blob.size();
   std::vector<float> blob32(blob.begin(), blob.end());
+  append(ts.ext);
   GD_HIP(hipMalloc(&ts.dev64, blob.size() * sizeof(double)));
   GD_HIP(hipMalloc(&ts.dev32, blob32.size() * sizeof(float)));
   GD_HIP(hipMemcpy(ts.dev64, blob.data(), blob.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -203,6 +217,7 @@ int build_tables(int basis, int n, int q, TableSet& ts)
     t.d1 = base + o;
   };
   fill(static_cast<double*>(ts.dev64), ts.t64);
+  fill(static_cast<double*>(ts.dev64) + len, ts.once64);
   fill(static_cast<float*>(ts.dev32), ts.t32);
   return GD_OK;
 }

@@ -77,7 +77,7 @@ int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStr
   a.bc_data = !a.bc_none && plan->bc_host.rank > 0;
   const Tables1D<T>* tab;
   if constexpr (std::is_same_v<T, double>) {
-    tab = &ts->t64;
+    tab = adv ? &ts->once64 : &ts->t64;  // mass applies keep the generic kernel's bits
     a.terms = plan->terms64;
     a.sigma_tab = static_cast<const FieldDev<double>*>(plan->fields64) + 3;
   } else {
