@@ -19,6 +19,17 @@
 // takes as many elements as fill its threads.  U and the sum V stay in LDS
 // through all passes, with the block's matrices.
 //
+// Rounding: M^-1 in the terms and M behind them amplify what the terms round.
+// So the matrices come from extended precision, rounded once; M is held in FP64
+// in units in which its entries round to almost nothing, and the passes with it
+// multiply in FP64 in either precision (an FP64 FMA costs what an FP32 one
+// does); a term's sum is formed apart and added once; with n = 2, where the
+// quadrature kernel has the fewest sums, the terms are formed in FP64 too.
+// Error against an extended-precision apply, in units of the generic kernel's:
+// FP64 up to 1.5 before, 0.05 to 0.64 now; FP32 up to 4.4 before (n = 3, q = 4
+// Lobatto), 0.2 to 1.1 now.  Times of FP32 applies before and now: 6D p = 2 82
+// and 88 us, 6D p = 1 10.7 and 12.8, 4D p = 3 22.2 and 23.3; FP64 unchanged.
+//
 // 6 x 6 x 6 x 5 x 5 x 5 elements, p = 2, q = 3, beta = (v, a), FP64 (315 MB in
 // and out): 163 us against 2,650 us for the generic kernel.  Bound by the waits
 // of the passes (60 % of the wave cycles), then VALU issue (60 us) and LDS.
@@ -39,9 +50,7 @@ struct Term {
   int a, b;            // axes; b: the matrix tb is along b (tb nullptr: none)
   int inflow;          // 0: no face; +1: the lower neighbour's upper end flows in, -1: the upper neighbour's lower end
   const T *ta, *tb, *tf;  // tf: [position along a][n]
-  T scale;             // times adv_coef or mass_coef
   int stride[6];       // strides of the other axes, ascending, then of a and b
-  int mass;            // 1: scaled by mass_coef
 };
 
 template <typename T>
@@ -50,8 +59,10 @@ struct Args {
   int M[6];
   pl::FastDiv dv[5];
   int periodic_mask;
-  T km, coef[kMaxTermsK];  // constant part of sigma; factors of the terms
-  const T *Mm, *b0, *b1;
+  double km;            // constant part of sigma
+  T coef[kMaxTermsK];   // factors of the terms
+  const double* Mm;
+  const T *b0, *b1;
   Term<T> t[kMaxTermsK];
 };
 
@@ -76,6 +87,7 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
 {
   using G = Geo<T, D, N>;
   constexpr int ND = G::ND, NS = G::NS, PITCH = G::PITCH, NT = G::NT, NN = N * N, TW = G::TW;
+  using C = std::conditional_t<N == 2, double, T>;  // the terms' arithmetic
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* U = reinterpret_cast<T*>(smem_raw);
   T* V = U + p.epb * PITCH;
@@ -147,9 +159,9 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
       const T* mk = mat + el * p.mpitch + k * TW;
       const int nb = face ? nbs[el * p.nterms + k] : -1;
       // the neighbour's line at the shared face, along b
-      T s[N];
+      C s[N];
 #pragma unroll
-      for (int j = 0; j < N; ++j) s[j] = T(0);
+      for (int j = 0; j < N; ++j) s[j] = C(0);
       if (nb >= 0) {
         const T* src = x + (int64_t)nb * ND + base;
         if constexpr (GLL) {
@@ -160,37 +172,37 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
           const T* be = tm.inflow > 0 ? p.b1 : p.b0;
 #pragma unroll
           for (int i = 0; i < N; ++i) {
-            const T c = be[i];
+            const C c = be[i];
 #pragma unroll
             for (int j = 0; j < N; ++j) s[j] += c * src[i * sa + j * sb];
           }
         }
       }
-      T S[N][N];
+      C S[N][N];
       const T* u = U + el * PITCH + base;
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int j = 0; j < N; ++j) S[i][j] = u[i * sa + j * sb];
       T* v = V + el * PITCH + base;
-      T W[N][N];
+      C W[N][N];
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int j = 0; j < N; ++j) W[i][j] = k == 0 ? p.km * S[i][j] : v[i * sa + j * sb];
+        for (int j = 0; j < N; ++j) W[i][j] = k == 0 ? (C)p.km * S[i][j] : v[i * sa + j * sb];
       if (two) {
-        T R[N][N], q[N];
+        C R[N][N], q[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-          q[j] = T(0);
+          q[j] = C(0);
 #pragma unroll
-          for (int i = 0; i < N; ++i) R[i][j] = T(0);
+          for (int i = 0; i < N; ++i) R[i][j] = C(0);
         }
 #pragma unroll
         for (int l = 0; l < N; ++l)
 #pragma unroll
           for (int j = 0; j < N; ++j) {
-            const T m = mk[NN + j * N + l];
+            const C m = mk[NN + j * N + l];
             q[j] += m * s[l];
 #pragma unroll
             for (int i = 0; i < N; ++i) R[i][j] += m * S[i][l];
@@ -202,34 +214,33 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
           for (int i = 0; i < N; ++i) S[i][j] = R[i][j];
         }
       }
+      C Z[N][N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const C f = face ? mk[2 * NN + i] : T(0);
+#pragma unroll
+        for (int j = 0; j < N; ++j) Z[i][j] = f * s[j];
+      }
 #pragma unroll
       for (int l = 0; l < N; ++l)
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          const T m = mk[i * N + l];
+          const C m = mk[i * N + l];
 #pragma unroll
-          for (int j = 0; j < N; ++j) W[i][j] += m * S[l][j];
+          for (int j = 0; j < N; ++j) Z[i][j] += m * S[l][j];
         }
-      if (face) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const T f = mk[2 * NN + i];
-#pragma unroll
-          for (int j = 0; j < N; ++j) W[i][j] += f * s[j];
-        }
-      }
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int j = 0; j < N; ++j) v[i * sa + j * sb] = W[i][j];
+        for (int j = 0; j < N; ++j) v[i * sa + j * sb] = (T)(W[i][j] + Z[i][j]);
     }
     __syncthreads();
   }
 
   // M along every axis, two at a time; the last pair goes out
-  pl::CPtr<T> M = (pl::CPtr<T>)p.Mm;
+  pl::CPtr<double> M = (pl::CPtr<double>)p.Mm;
   const T* from = p.nterms ? V : U;
-  const T first = p.nterms ? T(1) : p.km;
+  const double first = p.nterms ? 1.0 : p.km;
   constexpr int PAIRS = (D + 1) / 2;
   dev::static_for<0, PAIRS>([&](auto pr_) {
     constexpr int pr = decltype(pr_)::value;
@@ -244,7 +255,7 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
       const int lowd = r % sa, high = r / sa;  // axes below A, above Bx
       const int base = lowd + high * (sb * N);
       const T* src = (pr == 0 ? from : V) + el * PITCH + base;
-      T S[N][N], R[N][N];
+      double S[N][N], R[N][N];
 #pragma unroll
       for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -256,7 +267,7 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
       for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-          T q = M[i * N] * S[0][j];
+          double q = M[i * N] * S[0][j];
 #pragma unroll
           for (int l = 1; l < N; ++l) q += M[i * N + l] * S[l][j];
           R[i][j] = q;
@@ -266,7 +277,7 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
         for (int i = 0; i < N; ++i)
 #pragma unroll
           for (int j = 0; j < N; ++j) {
-            T q = M[j * N] * R[i][0];
+            double q = M[j * N] * R[i][0];
 #pragma unroll
             for (int l = 1; l < N; ++l) q += M[j * N + l] * R[i][l];
             S[i][j] = q;
@@ -282,13 +293,13 @@ __global__ void __launch_bounds__((Geo<T, D, N>::NT)) kron_kernel(Args<T> p, con
 #pragma unroll
         for (int i = 0; i < N; ++i)
 #pragma unroll
-          for (int j = 0; j < N; ++j) dst[i * sa + j * sb] = S[i][j];
+          for (int j = 0; j < N; ++j) dst[i * sa + j * sb] = (T)S[i][j];
       } else {
         T* dst = V + el * PITCH + base;
 #pragma unroll
         for (int i = 0; i < N; ++i)
 #pragma unroll
-          for (int j = 0; j < N; ++j) dst[i * sa + j * sb] = S[i][j];
+          for (int j = 0; j < N; ++j) dst[i * sa + j * sb] = (T)S[i][j];
       }
     }
     if constexpr (!last) __syncthreads();

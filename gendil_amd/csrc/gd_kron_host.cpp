@@ -24,7 +24,9 @@ struct State {
   bool adv_ok = false, mass_ok = false;
   std::vector<HostTerm> adv, mass;
   double sigma_const = 0.0;  // sum of sigma's constant terms
-  int64_t mm = 0;            // offset of the mass matrix
+  // offset of the mass matrix, M / unit; unit^dim goes into the factors of the terms
+  int64_t mm = 0;
+  double units = 1.0;
   // one allocation, kept from one set of coefficients to the next while they
   // fit: the values in FP64, then in FP32
   void* dev = nullptr;
@@ -42,12 +44,14 @@ void destroy_state(State* s)
 
 namespace {
 
-using Mat = std::vector<double>;  // n x n, row-major
+// Matrices are formed in extended precision and rounded once.
+using Ext = long double;
+using Mat = std::vector<Ext>;  // n x n, row-major
 
-// inverse by Gauss-Jordan with partial pivoting, in extended precision
+// inverse by Gauss-Jordan with partial pivoting
 Mat inverse(const Mat& a, int n)
 {
-  std::vector<long double> m((size_t)n * 2 * n, 0.0L);
+  Mat m((size_t)n * 2 * n, 0.0L);
   for (int i = 0; i < n; ++i) {
     for (int j = 0; j < n; ++j) m[i * 2 * n + j] = a[i * n + j];
     m[i * 2 * n + n + i] = 1.0L;
@@ -55,20 +59,43 @@ Mat inverse(const Mat& a, int n)
   for (int c = 0; c < n; ++c) {
     int p = c;
     for (int i = c + 1; i < n; ++i)
-      if (std::fabs((double)m[i * 2 * n + c]) > std::fabs((double)m[p * 2 * n + c])) p = i;
+      if (std::fabs(m[i * 2 * n + c]) > std::fabs(m[p * 2 * n + c])) p = i;
     for (int j = 0; j < 2 * n; ++j) std::swap(m[c * 2 * n + j], m[p * 2 * n + j]);
-    const long double d = m[c * 2 * n + c];
+    const Ext d = m[c * 2 * n + c];
     for (int j = 0; j < 2 * n; ++j) m[c * 2 * n + j] /= d;
     for (int i = 0; i < n; ++i) {
       if (i == c) continue;
-      const long double f = m[i * 2 * n + c];
+      const Ext f = m[i * 2 * n + c];
       for (int j = 0; j < 2 * n; ++j) m[i * 2 * n + j] -= f * m[c * 2 * n + j];
     }
   }
   Mat r((size_t)n * n);
   for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) r[i * n + j] = (double)m[i * 2 * n + n + j];
+    for (int j = 0; j < n; ++j) r[i * n + j] = m[i * 2 * n + n + j];
   return r;
+}
+
+// The unit in which M rounds best, M_00 / k for the k <= 64 with the smallest
+// rounding error: M multiplies along every axis, so an error of its entries adds
+// up over the axes, the same in every value.  Left over: at most 0.07 units in
+// the last place (n <= 5), against up to half a unit per axis.
+Ext mass_unit(const Mat& M)
+{
+  Ext best = -1.0L, unit = M[0];
+  for (int k = 1; k <= 64; ++k) {
+    const Ext u = M[0] / k;
+    Ext e = 0.0L;
+    for (const Ext v : M) {
+      const Ext d = (Ext)(double)(v / u) - v / u;
+      e += d * d;
+    }
+    e *= u * u;
+    if (best < 0.0L || e < best) {
+      best = e;
+      unit = u;
+    }
+  }
+  return unit;
 }
 
 const Entry* find(const gd_plan* plan)
@@ -155,39 +182,43 @@ int refresh(const gd_plan* plan)
   const int n = plan->desc.order + 1, q = plan->desc.num_quad;
   const TableSet* ts = find_tables(plan, n, q);
   if (!ts || q < n) return GD_OK;  // M is singular with fewer points than nodes
-  auto gram = [&](const std::vector<double>& L, const double* f) {  // L^T W f B
-    Mat m((size_t)n * n, 0.0);
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j)
-        for (int k = 0; k < q; ++k) m[i * n + j] += ts->w[k] * (f ? f[k] : 1.0) * L[k * n + i] * ts->B[k * n + j];
+  const RuleTables<Ext>& t1 = ts->ext;
+  auto gram = [&](const Mat& L, const double* f) {  // L^T W f B
+    Mat m((size_t)n * n, 0.0L);
+    for (int k = 0; k < q; ++k) {
+      const Ext wf = t1.w[k] * (f ? f[k] : 1.0);
+      for (int i = 0; i < n; ++i)
+        for (int j = 0; j < n; ++j) m[i * n + j] += wf * L[k * n + i] * t1.B[k * n + j];
+    }
     return m;
   };
-  const Mat M = gram(ts->B, nullptr), Mi = inverse(M, n);
+  const Mat M = gram(t1.B, nullptr), Mi = inverse(M, n);
   std::vector<double> blob;
   auto put = [&](const Mat& m) {
     const int64_t at = (int64_t)blob.size();
-    blob.insert(blob.end(), m.begin(), m.end());
+    for (const Ext v : m) blob.push_back((double)v);
     return at;
   };
   auto times = [&](const Mat& m) {  // M^-1 m, m with n rows
     const int cols = (int)m.size() / n;
-    Mat r(m.size(), 0.0);
+    Mat r(m.size(), 0.0L);
     for (int i = 0; i < n; ++i)
-      for (int j = 0; j < cols; ++j) {
-        long double s = 0.0L;
-        for (int k = 0; k < n; ++k) s += (long double)Mi[i * n + k] * m[k * cols + j];
-        r[i * cols + j] = (double)s;
-      }
+      for (int k = 0; k < n; ++k)
+        for (int j = 0; j < cols; ++j) r[i * cols + j] += Mi[i * n + k] * m[k * cols + j];
     return r;
   };
-  st.mm = put(M);
+  const Ext unit = mass_unit(M);
+  Mat Mu(M);
+  for (Ext& v : Mu) v /= unit;
+  st.mm = put(Mu);
+  st.units = (double)std::pow(unit, D);
   // factor matrices M^-1 B^T W f B per position along an axis
   auto factor = [&](int axis, const double* v, double scale) {
     const int64_t at = (int64_t)blob.size();
     for (int64_t e = 0; e < plan->desc.sizes[axis]; ++e) {
-      Mat f(q);
+      std::vector<double> f(q);
       for (int k = 0; k < q; ++k) f[k] = scale * v[e * (q + 2) + k];
-      put(times(gram(ts->B, f.data())));
+      put(times(gram(t1.B, f.data())));
     }
     return at;
   };
@@ -258,12 +289,12 @@ int refresh(const gd_plan* plan)
     for (int64_t e = 0; e < Mc; ++e) {
       const double* v = f.axis == c ? f.v.data() + e * (q + 2) : nullptr;
       const double cst = f.axis < 0 ? f.v[0] : 1.0;
-      Mat m = gram(ts->Gb, v);
-      for (double& s : m) s *= -cst;
+      Mat m = gram(t1.Gb, v);
+      for (Ext& s : m) s *= -cst;
       // own face at the outflow end: there with a neighbour or inflow data
       const bool edge = !per && (neg ? e == 0 : e == Mc - 1);
       if (!(edge && plan->bc_mode == GD_BC_NONE)) {
-        const std::vector<double>& be = neg ? ts->b0 : ts->b1;
+        const Mat& be = neg ? t1.b0 : t1.b1;
         const double bo = (v ? v[neg ? q : q + 1] : 1.0) * cst * (neg ? -1.0 : 1.0);
         for (int i = 0; i < n; ++i)
           for (int j = 0; j < n; ++j) m[i * n + j] += bo * be[i] * be[j];
@@ -272,7 +303,7 @@ int refresh(const gd_plan* plan)
       // inflow end: -beta b0 (lower face) or +beta b1 (upper face) on the neighbour's trace
       const double bi = (v ? v[neg ? q + 1 : q] : 1.0) * cst * (neg ? 1.0 : -1.0);
       Mat col(n);
-      for (int i = 0; i < n; ++i) col[i] = bi * (neg ? ts->b1[i] : ts->b0[i]);
+      for (int i = 0; i < n; ++i) col[i] = bi * (neg ? t1.b1[i] : t1.b0[i]);
       const Mat fc = times(col);
       fv.insert(fv.end(), fc.begin(), fc.end());
     }
@@ -332,7 +363,7 @@ int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStr
   const Tables1D<T>* tab;
   if constexpr (std::is_same_v<T, double>) {
     base = st.f64();
-    tab = &ts->t64;
+    tab = &ts->once64;
   } else {
     base = st.f32();
     tab = &ts->t32;
@@ -346,8 +377,9 @@ int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStr
     if (plan->desc.periodic[d]) a.periodic_mask |= 1 << d;
     detJ *= plan->desc.h[d];
   }
-  a.km = mass ? (T)((double)mass_coef * detJ * st.sigma_const) : T(0);
-  a.Mm = base + st.mm;
+  detJ *= st.units;
+  a.km = mass ? (double)mass_coef * detJ * st.sigma_const : 0.0;
+  a.Mm = st.f64() + st.mm;
   a.b0 = tab->b0;
   a.b1 = tab->b1;
   a.nterms = 0;

@@ -1,10 +1,13 @@
-"""Tables rounded once where a kernel mirrors half of them: the mass part of a
-one-cell advection step against the same operator in extended precision."""
+"""Tables rounded once where a kernel mirrors half of them or multiplies by
+products of them: the mass part of a one-cell advection step, and one-cell mass
+applies of the 4D-6D Kronecker kernel, against the same operator in extended
+precision."""
 import numpy as np
 import pytest
 import torch
 
 import gendil_amd as G
+from test_gpu_kron import KRON, SHAPES
 from test_gpu_plane import PAIRS, PLANE
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +83,20 @@ def test_plane_kernel(n, q, basis):
                                      adv_coef=2.0**-80)
     op.plan.set_variant(torch.float64, PLANE)
     assert apply_error(op, torch.float64, 3, n, mass_matrix(basis, n, q)) <= 7 * U
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
+@pytest.mark.parametrize("basis", [0, 1])
+@pytest.mark.parametrize("D,n", SHAPES)
+def test_kronecker_kernel(D, n, basis, dtype):
+    """D contractions of n products with a mass matrix that rounds to almost nothing, and one factor: sqrt(D n + 1) U in
+    FP64 as a walk.  FP32: FP64 sums, stored (D + 1) / 2 times.  With M rounded entry by entry its error is the same in
+    every value and axis."""
+    op = G.MakeMassFiniteElementOperator(one_cell(D, basis, n), G.MakeIntegrationRule(n), None)
+    op.plan.set_variant(dtype, KRON)
+    assert op.plan.query_variant(dtype, 1.0, 0.0) == KRON
+    u = U if dtype == torch.float64 else 2.0**-24
+    bound = (D * n + 1) ** 0.5 if dtype == torch.float64 else ((D + 1) // 2) ** 0.5
+    err = apply_error(op, dtype, D, n, mass_matrix(basis, n, n)) / u
+    print(f"error {err:.2f} U, bound {bound:.2f} U")
+    assert err <= bound
