@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -46,32 +47,34 @@ namespace {
 
 // Matrices are formed in extended precision and rounded once.
 using Ext = long double;
-using Mat = std::vector<Ext>;  // n x n, row-major
+constexpr int kMaxN = 5;  // nodes of any instance
+using Table = std::vector<Ext>;
+using Mat = std::array<Ext, kMaxN * kMaxN>;  // n x n or n x 1, row-major
 
 // inverse by Gauss-Jordan with partial pivoting
 Mat inverse(const Mat& a, int n)
 {
-  Mat m((size_t)n * 2 * n, 0.0L);
+  Ext m[kMaxN][2 * kMaxN] = {};
   for (int i = 0; i < n; ++i) {
-    for (int j = 0; j < n; ++j) m[i * 2 * n + j] = a[i * n + j];
-    m[i * 2 * n + n + i] = 1.0L;
+    for (int j = 0; j < n; ++j) m[i][j] = a[i * n + j];
+    m[i][n + i] = 1.0L;
   }
   for (int c = 0; c < n; ++c) {
     int p = c;
     for (int i = c + 1; i < n; ++i)
-      if (std::fabs(m[i * 2 * n + c]) > std::fabs(m[p * 2 * n + c])) p = i;
-    for (int j = 0; j < 2 * n; ++j) std::swap(m[c * 2 * n + j], m[p * 2 * n + j]);
-    const Ext d = m[c * 2 * n + c];
-    for (int j = 0; j < 2 * n; ++j) m[c * 2 * n + j] /= d;
+      if (std::fabs(m[i][c]) > std::fabs(m[p][c])) p = i;
+    for (int j = 0; j < 2 * n; ++j) std::swap(m[c][j], m[p][j]);
+    const Ext d = m[c][c];
+    for (int j = 0; j < 2 * n; ++j) m[c][j] /= d;
     for (int i = 0; i < n; ++i) {
       if (i == c) continue;
-      const Ext f = m[i * 2 * n + c];
-      for (int j = 0; j < 2 * n; ++j) m[i * 2 * n + j] -= f * m[c * 2 * n + j];
+      const Ext f = m[i][c];
+      for (int j = 0; j < 2 * n; ++j) m[i][j] -= f * m[c][j];
     }
   }
-  Mat r((size_t)n * n);
+  Mat r{};
   for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) r[i * n + j] = m[i * 2 * n + n + j];
+    for (int j = 0; j < n; ++j) r[i * n + j] = m[i][n + j];
   return r;
 }
 
@@ -79,14 +82,14 @@ Mat inverse(const Mat& a, int n)
 // rounding error: M multiplies along every axis, so an error of its entries adds
 // up over the axes, the same in every value.  Left over: at most 0.07 units in
 // the last place (n <= 5), against up to half a unit per axis.
-Ext mass_unit(const Mat& M)
+Ext mass_unit(const Mat& M, int n)
 {
   Ext best = -1.0L, unit = M[0];
   for (int k = 1; k <= 64; ++k) {
     const Ext u = M[0] / k;
     Ext e = 0.0L;
-    for (const Ext v : M) {
-      const Ext d = (Ext)(double)(v / u) - v / u;
+    for (int i = 0; i < n * n; ++i) {
+      const Ext v = M[i] / u, d = (Ext)(double)v - v;
       e += d * d;
     }
     e *= u * u;
@@ -183,8 +186,8 @@ int refresh(const gd_plan* plan)
   const TableSet* ts = find_tables(plan, n, q);
   if (!ts || q < n) return GD_OK;  // M is singular with fewer points than nodes
   const RuleTables<Ext>& t1 = ts->ext;
-  auto gram = [&](const Mat& L, const double* f) {  // L^T W f B
-    Mat m((size_t)n * n, 0.0L);
+  auto gram = [&](const Table& L, const double* f) {  // L^T W f B
+    Mat m{};
     for (int k = 0; k < q; ++k) {
       const Ext wf = t1.w[k] * (f ? f[k] : 1.0);
       for (int i = 0; i < n; ++i)
@@ -194,31 +197,30 @@ int refresh(const gd_plan* plan)
   };
   const Mat M = gram(t1.B, nullptr), Mi = inverse(M, n);
   std::vector<double> blob;
-  auto put = [&](const Mat& m) {
-    const int64_t at = (int64_t)blob.size();
-    for (const Ext v : m) blob.push_back((double)v);
+  auto put = [&](std::vector<double>& to, const Mat& m, int count) {
+    const int64_t at = (int64_t)to.size();
+    for (int i = 0; i < count; ++i) to.push_back((double)m[i]);
     return at;
   };
-  auto times = [&](const Mat& m) {  // M^-1 m, m with n rows
-    const int cols = (int)m.size() / n;
-    Mat r(m.size(), 0.0L);
+  auto times = [&](const Mat& m, int cols) {  // M^-1 m
+    Mat r{};
     for (int i = 0; i < n; ++i)
       for (int k = 0; k < n; ++k)
         for (int j = 0; j < cols; ++j) r[i * cols + j] += Mi[i * n + k] * m[k * cols + j];
     return r;
   };
-  const Ext unit = mass_unit(M);
+  const Ext unit = mass_unit(M, n);
   Mat Mu(M);
   for (Ext& v : Mu) v /= unit;
-  st.mm = put(Mu);
+  st.mm = put(blob, Mu, n * n);
   st.units = (double)std::pow(unit, D);
   // factor matrices M^-1 B^T W f B per position along an axis
   auto factor = [&](int axis, const double* v, double scale) {
     const int64_t at = (int64_t)blob.size();
+    std::vector<double> f(q);
     for (int64_t e = 0; e < plan->desc.sizes[axis]; ++e) {
-      std::vector<double> f(q);
       for (int k = 0; k < q; ++k) f[k] = scale * v[e * (q + 2) + k];
-      put(times(gram(t1.B, f.data())));
+      put(blob, times(gram(t1.B, f.data()), n), n * n);
     }
     return at;
   };
@@ -284,30 +286,40 @@ int refresh(const gd_plan* plan)
     t.b = f.axis >= 0 && f.axis != c ? f.axis : (c == 0 ? 1 : 0);
     t.inflow = neg ? -1 : 1;
     t.scale = 1.0 / plan->desc.h[c];
-    Mat fv;
+    std::vector<double> fv;
     t.ta = (int64_t)blob.size();
+    // a component that does not vary along its own axis has one matrix, and one
+    // more at a boundary it skips
+    Mat A, fc;
+    bool same = false, was = false;
     for (int64_t e = 0; e < Mc; ++e) {
       const double* v = f.axis == c ? f.v.data() + e * (q + 2) : nullptr;
       const double cst = f.axis < 0 ? f.v[0] : 1.0;
-      Mat m = gram(t1.Gb, v);
-      for (Ext& s : m) s *= -cst;
       // own face at the outflow end: there with a neighbour or inflow data
-      const bool edge = !per && (neg ? e == 0 : e == Mc - 1);
-      if (!(edge && plan->bc_mode == GD_BC_NONE)) {
-        const Mat& be = neg ? t1.b0 : t1.b1;
-        const double bo = (v ? v[neg ? q : q + 1] : 1.0) * cst * (neg ? -1.0 : 1.0);
-        for (int i = 0; i < n; ++i)
-          for (int j = 0; j < n; ++j) m[i * n + j] += bo * be[i] * be[j];
+      const bool own = per || plan->bc_mode != GD_BC_NONE || (neg ? e != 0 : e != Mc - 1);
+      if (v || !same || own != was) {
+        Mat m = gram(t1.Gb, v);
+        for (Ext& s : m) s *= -cst;
+        if (own) {
+          const Table& be = neg ? t1.b0 : t1.b1;
+          const double bo = (v ? v[neg ? q : q + 1] : 1.0) * cst * (neg ? -1.0 : 1.0);
+          for (int i = 0; i < n; ++i)
+            for (int j = 0; j < n; ++j) m[i * n + j] += bo * be[i] * be[j];
+        }
+        A = times(m, n);
+        // inflow end: -beta b0 (lower face) or +beta b1 (upper face) on the neighbour's trace
+        const double bi = (v ? v[neg ? q + 1 : q] : 1.0) * cst * (neg ? 1.0 : -1.0);
+        Mat col{};
+        for (int i = 0; i < n; ++i) col[i] = bi * (neg ? t1.b1[i] : t1.b0[i]);
+        fc = times(col, 1);
+        same = true;
+        was = own;
       }
-      put(times(m));
-      // inflow end: -beta b0 (lower face) or +beta b1 (upper face) on the neighbour's trace
-      const double bi = (v ? v[neg ? q + 1 : q] : 1.0) * cst * (neg ? 1.0 : -1.0);
-      Mat col(n);
-      for (int i = 0; i < n; ++i) col[i] = bi * (neg ? t1.b1[i] : t1.b0[i]);
-      const Mat fc = times(col);
-      fv.insert(fv.end(), fc.begin(), fc.end());
+      put(blob, A, n * n);
+      put(fv, fc, n);
     }
-    t.tf = put(fv);
+    t.tf = (int64_t)blob.size();
+    blob.insert(blob.end(), fv.begin(), fv.end());
     if (f.axis >= 0 && f.axis != c) t.tb = factor(f.axis, f.v.data(), 1.0);
     st.adv.push_back(t);
   }
