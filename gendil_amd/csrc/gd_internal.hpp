@@ -123,8 +123,7 @@ struct RuleTables {
 // operator are compared with GenDiL's).
 struct TableSet : RuleTables<double> {
   int n = 0, q = 0;
-  void* dev64 = nullptr;  // contiguous device block (double)
-  void* dev32 = nullptr;  // contiguous device block (float)
+  void* dev = nullptr;  // one device block
   Tables1D<double> t64{}, once64{};
   Tables1D<float> t32{};
   RuleTables<long double> ext;

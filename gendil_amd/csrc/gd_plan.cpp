@@ -182,7 +182,8 @@ int build_tables(int basis, int n, int q, TableSet& ts)
   ts.q = q;
   compute_tables<double>(basis, n, q, ts);
   compute_tables<long double>(basis, n, q, ts.ext);
-  // device upload: B | Gq | b0 | b1 | w | xq | Gb | d0 | d1, then (FP64) the same rounded once
+  // device upload, one block: B | Gq | b0 | b1 | w | xq | Gb | d0 | d1, the same
+  // rounded once, and the first in FP32
   std::vector<double> blob;
   auto append = [&](const auto& t) {
     for (const auto* v : {&t.B, &t.Gq, &t.b0, &t.b1, &t.w, &t.xq, &t.Gb, &t.d0, &t.d1})
@@ -190,12 +191,13 @@ int build_tables(int basis, int n, int q, TableSet& ts)
   };
   append(static_cast<const RuleTables<double>&>(ts));
   const size_t len = blob.size();
-  std::vector<float> blob32(blob.begin(), blob.end());
+  const std::vector<float> blob32(blob.begin(), blob.end());
   append(ts.ext);
-  GD_HIP(hipMalloc(&ts.dev64, blob.size() * sizeof(double)));
-  GD_HIP(hipMalloc(&ts.dev32, blob32.size() * sizeof(float)));
-  GD_HIP(hipMemcpy(ts.dev64, blob.data(), blob.size() * sizeof(double), hipMemcpyHostToDevice));
-  GD_HIP(hipMemcpy(ts.dev32, blob32.data(), blob32.size() * sizeof(float), hipMemcpyHostToDevice));
+  blob.resize(2 * len + (len + 1) / 2);
+  std::memcpy(blob.data() + 2 * len, blob32.data(), len * sizeof(float));
+  GD_HIP(hipMalloc(&ts.dev, blob.size() * sizeof(double)));
+  GD_HIP(hipMemcpy(ts.dev, blob.data(), blob.size() * sizeof(double), hipMemcpyHostToDevice));
+  double* base64 = static_cast<double*>(ts.dev);
   auto fill = [&](auto* base, auto& t) {
     size_t o = 0;
     t.B = base + o;
@@ -216,9 +218,9 @@ int build_tables(int basis, int n, int q, TableSet& ts)
     o += n;
     t.d1 = base + o;
   };
-  fill(static_cast<double*>(ts.dev64), ts.t64);
-  fill(static_cast<double*>(ts.dev64) + len, ts.once64);
-  fill(static_cast<float*>(ts.dev32), ts.t32);
+  fill(base64, ts.t64);
+  fill(base64 + len, ts.once64);
+  fill(reinterpret_cast<float*>(base64 + 2 * len), ts.t32);
   return GD_OK;
 }
 
@@ -463,8 +465,7 @@ template Params<float> make_params<float>(const gd_plan*, const TableSet*, float
 gd_plan::~gd_plan()
 {
   for (gd::TableSet* t : tables) {
-    if (t->dev64) (void)hipFree(t->dev64);
-    if (t->dev32) (void)hipFree(t->dev32);
+    if (t->dev) (void)hipFree(t->dev);
     delete t;
   }
   if (dof_offset_dev) (void)hipFree(dof_offset_dev);
