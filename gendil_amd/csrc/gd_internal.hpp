@@ -86,7 +86,6 @@ struct Params {
   // coefficients
   int beta_kind;            // gd_beta_kind
   const FieldDev<T>* beta;  // [dim] (separable)
-  const FieldTerms<T>* terms;  // 3D plans
   const FieldDev<T>* sigma;
   const FieldDev<T>* bc;
   int bc_mode;

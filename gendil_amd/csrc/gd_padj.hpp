@@ -634,14 +634,9 @@ int launch_adjoint(AdjArgs& a, bool grad, const double* x, double* y, hipStream_
   while (a.epb > 2 && (int64_t)a.epb * 512 > a.E) a.epb = (a.epb + 1) / 2;
   a.num_blocks = (int)((a.E + a.epb - 1) / a.epb);
   const size_t lds = a.epb * per;
-  constexpr size_t most = (size_t)G::EPB * (Q * G::GP + G::GZ) * sizeof(double);
-  static_assert(most <= 160 * 1024, "LDS of one block");
-  if (lds > 64 * 1024) {
-    static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(grad_plane_kernel<N, Q, GLL>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
-    GD_HIP(attr);
-  }
+  constexpr int tr = Q * G::TP + 2 * G::TZ, gr = Q * G::GP + G::GZ;
+  constexpr size_t most = (size_t)G::EPB * (tr > gr ? tr : gr) * sizeof(double);
+  static_assert(most <= 64 * 1024, "LDS of one block without an attribute");
   if (grad) hipLaunchKernelGGL((grad_plane_kernel<N, Q, GLL>), dim3((unsigned)a.num_blocks), dim3(G::NT), lds, s, a, x, y);
   else hipLaunchKernelGGL((transpose_plane_kernel<N, Q, GLL>), dim3((unsigned)a.num_blocks), dim3(G::NT), lds, s, a, x, y);
   GD_HIP(hipGetLastError());

@@ -426,11 +426,9 @@ Params<T> make_params(const gd_plan* p, const TableSet* ts, T mass_coef, T adv_c
   if constexpr (std::is_same_v<T, double>) {
     k.tab = ts->t64;
     k.beta = static_cast<const FieldDev<double>*>(p->fields64);
-    k.terms = p->terms64;
   } else {
     k.tab = ts->t32;
     k.beta = static_cast<const FieldDev<float>*>(p->fields32);
-    k.terms = p->terms32;
   }
   k.sigma = k.beta + D;
   k.bc = (p->bc_mode == GD_BC_INFLOW && p->bc_host.rank > 0) ? k.beta + D + 1 : nullptr;

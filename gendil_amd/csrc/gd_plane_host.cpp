@@ -22,7 +22,7 @@ const Entry* find(int N, int Q)
 }
 
 // 3D, uniform order; element and neighbour numbers in 32 bits
-const Entry* serving(const gd_plan* plan, bool adv)
+const Entry* serving(const gd_plan* plan)
 {
   if (plan->dim != 3 || plan->padapt || plan->E >= (int64_t)1 << 31) return nullptr;
   return find(plan->desc.order + 1, plan->desc.num_quad);
@@ -31,9 +31,9 @@ const Entry* serving(const gd_plan* plan, bool adv)
 }  // namespace
 
 template <typename T>
-bool available(const gd_plan* plan, bool adv, bool /*mass*/)
+bool available(const gd_plan* plan, bool /*adv*/, bool /*mass*/)
 {
-  return serving(plan, adv) != nullptr;
+  return serving(plan) != nullptr;
 }
 
 template <typename T>
@@ -47,7 +47,7 @@ template <typename T>
 int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStream_t s)
 {
   const bool adv = adv_coef != T(0);
-  const Entry* en = serving(plan, adv);
+  const Entry* en = serving(plan);
   if (!en) return GD_ERR_UNSUPPORTED;
   const TableSet* ts = find_tables(plan, en->N, en->Q);
   Args<T> a;
