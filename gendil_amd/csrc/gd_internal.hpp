@@ -113,19 +113,20 @@ struct RuleTables {
 };
 
 // The tables as FP64 arithmetic gives them (a few units off in the last place),
-// and the same from extended precision.  Kernels that hold half of a table and
-// mirror it, or products of tables, read the latter, rounded once: there an
-// entry's error meets itself in every sum (n = 3..5 on Lobatto nodes, 3D apply:
-// up to 1.5 times the generic kernel's error against an extended-precision
-// apply with the former, at most 0.7 times with the latter).  The others keep
-// the former and with it their bits (iteration counts of a solve on a mass
-// operator are compared with GenDiL's).
+// and, on Lobatto nodes, the same from extended precision.  Kernels that hold
+// half of a table and mirror it, or products of tables, read the latter, rounded
+// once: there an entry's error meets itself in every sum (n = 3..5, 3D apply: up
+// to 1.5 times the generic kernel's error against an extended-precision apply
+// with the former, at most 0.7 times with the latter).  On Legendre nodes these
+// kernels were no further off than the generic one (0.6 to 1.0 times) and read
+// the former, as the other kernels do, which keep their bits with it (iteration
+// counts of a solve on a mass operator are compared with GenDiL's).
 struct TableSet : RuleTables<double> {
   int n = 0, q = 0;
   void* dev = nullptr;  // one device block
   Tables1D<double> t64{}, once64{};
   Tables1D<float> t32{};
-  RuleTables<long double> ext;
+  RuleTables<long double> ext;  // what once64 rounds
 };
 
 struct HostField {

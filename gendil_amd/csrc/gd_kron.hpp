@@ -20,15 +20,16 @@
 // through all passes, with the block's matrices.
 //
 // Rounding: M^-1 in the terms and M behind them amplify what the terms round.
-// So the matrices come from extended precision, rounded once; M is held in FP64
+// So the matrices are formed in extended precision, rounded once; M is held in FP64
 // in units in which its entries round to almost nothing, and the passes with it
 // multiply in FP64 in either precision (an FP64 FMA costs what an FP32 one
 // does); a term's sum is formed apart and added once; with n = 2, where the
 // quadrature kernel has the fewest sums, the terms are formed in FP64 too.
 // Error against an extended-precision apply, in units of the generic kernel's:
-// FP64 up to 1.5 before, 0.05 to 0.64 now; FP32 up to 4.4 before (n = 3, q = 4
-// Lobatto), 0.2 to 1.1 now.  Times of FP32 applies before and now: 6D p = 2 82
-// and 88 us, 6D p = 1 10.7 and 12.8, 4D p = 3 22.2 and 23.3; FP64 unchanged.
+// FP64 Lobatto up to 1.5 before, 0.05 to 0.64 now (Legendre, on the generic
+// kernel's tables, 0.8 to 1.1); FP32 up to 4.4 before (n = 3, q = 4 Lobatto), 0.2
+// to 1.1 now.  FP32 applies before and now: 6D p = 2 82 and 88 us, 6D p = 1 10.9
+// and 13.0, 4D p = 3 22.3 and 23.6; FP64 unchanged.
 //
 // 6 x 6 x 6 x 5 x 5 x 5 elements, p = 2, q = 3, beta = (v, a), FP64 (315 MB in
 // and out): 163 us against 2,650 us for the generic kernel.  Bound by the waits

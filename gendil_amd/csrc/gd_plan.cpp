@@ -181,7 +181,14 @@ int build_tables(int basis, int n, int q, TableSet& ts)
   ts.n = n;
   ts.q = q;
   compute_tables<double>(basis, n, q, ts);
-  compute_tables<long double>(basis, n, q, ts.ext);
+  if (basis == GD_BASIS_GLL) {
+    compute_tables<long double>(basis, n, q, ts.ext);
+  } else {
+    const RuleTables<double>& t = ts;
+    auto widen = [](const std::vector<double>& v) { return std::vector<long double>(v.begin(), v.end()); };
+    ts.ext = {widen(t.B),  widen(t.Gq), widen(t.b0), widen(t.b1), widen(t.w),
+              widen(t.xq), widen(t.Gb), widen(t.d0), widen(t.d1)};
+  }
   // device upload, one block: B | Gq | b0 | b1 | w | xq | Gb | d0 | d1, the same
   // rounded once, and the first in FP32
   std::vector<double> blob;

