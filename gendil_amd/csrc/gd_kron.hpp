@@ -39,6 +39,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gd_plane.hpp"
+#include "gd_sizing.hpp"
 
 namespace gd {
 namespace kron {
@@ -312,11 +313,12 @@ int launch(Args<T>& a, const T* x, T* y, hipStream_t s)
 {
   using G = Geo<T, D, N>;
   a.mpitch = (a.nterms * G::TW) | 1;
-  a.epb = G::EPB;
-  while (a.epb > 1 && (int64_t)a.epb * 512 > a.E) a.epb = (a.epb + 1) / 2;
-  a.num_blocks = (int)(((int64_t)a.E + a.epb - 1) / a.epb);
-  const size_t lds = (size_t)a.epb * (2 * G::PITCH + a.mpitch) * sizeof(T) + (size_t)a.epb * a.nterms * sizeof(int);
   auto kern = kron_kernel<T, D, N, GLL>;
+  static const int resident = blocks_per_cu(kern, G::NT);
+  const size_t per = (2 * G::PITCH + a.mpitch) * sizeof(T) + a.nterms * sizeof(int);
+  a.epb = elements_per_block(a.E, 1, G::EPB, per, resident);
+  a.num_blocks = (int)(((int64_t)a.E + a.epb - 1) / a.epb);
+  const size_t lds = a.epb * per;
   if (lds > 160 * 1024) return GD_ERR_UNSUPPORTED;
   if (lds > 64 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

@@ -38,9 +38,10 @@ template <typename T>
 bool available(const gd_plan* plan, bool adv, bool mass);
 
 // Whether it is the faster one: always, except that the FP64 advection apply
-// with n = 5, q = 6 spills registers and a small mesh cannot hide it (measured
-// against the generic kernel: 216 elements 25.8 against 23.1 us, 1,000 25 and
-// 30 us, 1,728 22 and 26 us; half its time from 46,656 on).
+// with n = 5, q = 6 spills registers and a small mesh cannot hide it (generic
+// kernel against this: 216 elements 19 and 24 us with an affine field, 29 and 24
+// with one over two coordinates; 1,000 20 and 22, 29 and 21; 1,728 22 and 22, 31
+// and 21; 15,625 87 and 77, 122 and 58).
 template <typename T>
 bool preferred(const gd_plan* plan, bool adv);
 

@@ -4,6 +4,7 @@
 
 #include "gd_plane.hpp"
 #include "gd_plane_api.hpp"
+#include "gd_sizing.hpp"
 
 namespace gd {
 namespace pl {
@@ -16,11 +17,13 @@ int launch_kind(Args<T>& a, const T* x, T* y, hipStream_t s)
   const size_t per = (size_t)(G::PL * G::PITCH + a.spitch) * sizeof(T);
   // full blocks, unless the coefficients' samples leave too little LDS for two
   // blocks a CU or the mesh is too small for two blocks a CU
-  a.epb = G::EPB;
-  while (a.epb > 4 && ((int64_t)a.epb * 512 > a.E || (size_t)a.epb * per > 80 * 1024)) a.epb = (a.epb + 1) / 2;
+  auto kern = plane_kernel<T, N, Q, ADV, GLL, FIELD>;
+  static const int resident = blocks_per_cu(kern, G::NT);
+  int most = G::EPB;
+  while (most > 4 && (size_t)most * per > 80 * 1024) most = (most + 1) / 2;
+  a.epb = elements_per_block(a.E, 4, most, per, resident);
   a.num_blocks = (int)((a.E + a.epb - 1) / a.epb);
   const size_t lds = a.epb * per;
-  auto kern = plane_kernel<T, N, Q, ADV, GLL, FIELD>;
   if (lds > 160 * 1024) return GD_ERR_UNSUPPORTED;
   if (lds > 64 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

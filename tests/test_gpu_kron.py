@@ -73,6 +73,12 @@ def test_advection_boundaries_and_one_cell_axes(D, bc, kind):
     run(D, 2, 3, "L", [1, 4, 1, 3, 2, 1][:D], True, beta, bc, None, 0.0, -0.5)
 
 
+@pytest.mark.parametrize("D,n,sizes", [(4, 4, [5, 5, 5, 6]), (4, 4, [8, 7, 7, 8]), (4, 3, [8, 8, 8, 7]), (5, 3, [5, 4, 5, 4, 4])], ids=str)
+def test_block_sizes_of_one_round(D, n, sizes):
+    """Meshes whose elements per block follow the blocks that are resident at once."""
+    run(D, n, n, "L", sizes, False, mixed_field(D), None, None, 0.0, 1.0)
+
+
 @pytest.mark.parametrize("D,n,q", [(4, 5, 6), (5, 3, 4), (6, 3, 4)])
 def test_mass(D, n, q):
     for sigma in (None, sigma_field("poly", D)):

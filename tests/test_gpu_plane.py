@@ -78,6 +78,13 @@ def test_advection_sizes_and_boundaries(sizes, periodic, kind, bc):
     check(space(sizes, 2, "L", periodic), 4, torch.float64, field(kind), bc, None, 0.0, 1.0)
 
 
+@pytest.mark.parametrize("n,q", [(4, 6), (5, 5), (5, 6)])
+@pytest.mark.parametrize("sizes", [(13, 11, 12), (13, 11, 17), (19, 17, 13), (25, 21, 20)], ids=str)
+def test_block_sizes_of_one_round(n, q, sizes):
+    """Meshes whose elements per block follow the blocks that are resident at once: 4, 5, 9 and 21 elements."""
+    check(space(sizes, n - 1, "L", [False, True, False]), q, torch.float64, field("mixed"), "none", None, 0.0, 1.0)
+
+
 @pytest.mark.parametrize("n,q", [(2, 4), (3, 5), (4, 6), (5, 6)])
 @pytest.mark.parametrize("sizes", [(1, 1, 1), (9, 5, 3)], ids=str)
 def test_mass(n, q, sizes):
