@@ -101,7 +101,7 @@ int highdim_choice(const gd_plan* plan, bool adv, bool mass)
   if (tuned == 0) return 0;
   if (tuned == kron::kVariant && kron::available(plan, adv, mass)) return kron::kVariant;
   if (n2k::available<T>(plan, adv, mass)) return n2k::kVariant;
-  return kron::preferred(plan, adv, mass) ? kron::kVariant : 0;
+  return kron::preferred<T>(plan, adv, mass) ? kron::kVariant : 0;
 }
 
 // The register-resident kernel covers 3D GLL elements with q = p+1 and

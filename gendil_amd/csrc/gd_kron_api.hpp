@@ -39,6 +39,7 @@ int refresh(const gd_plan* plan);
 // Whether the kernel serves these coefficients, and whether it is the default
 // for them.
 bool available(const gd_plan* plan, bool adv, bool mass);
+template <typename T>
 bool preferred(const gd_plan* plan, bool adv, bool mass);
 
 template <typename T>

@@ -354,12 +354,30 @@ bool available(const gd_plan* plan, bool adv, bool mass)
   return st && (st->adv_ok || st->mass_ok) && (!adv || st->adv_ok) && (!mass || st->mass_ok);
 }
 
+template <typename T>
 bool preferred(const gd_plan* plan, bool adv, bool mass)
 {
   // a handful of elements (unit tests, debugging runs) stay on the generic
   // kernel, which takes the quadrature as it is written
-  return plan->E > 64 && available(plan, adv, mass);
+  if (plan->E <= 64 || !available(plan, adv, mass)) return false;
+  // Mass alone with a variable sigma and q = n: the generic kernel interpolates
+  // little, and this one holds few elements of these sizes in a CU.  Generic
+  // against this, sigma of two terms, us: FP64 4D n = 4 625 elements 8.5 and 8.3,
+  // 1,080 9.1 and 9.7, 8,100 26 and 32, 50,176 124 and 176 (4,096 17 and 16); FP64
+  // 4D n = 5 256 8.5 and 10, 1,080 11 and 11, 2,058 19 and 16; FP32 5D n = 4 625
+  // 10.4 and 10.6, 2,058 20 and 24, 20,736 132 and 140.  All others gain at every
+  // size.
+  const int n = plan->desc.order + 1;
+  if (!adv && plan->desc.num_quad == n && !plan->kron_state->mass.empty()) {
+    if (sizeof(T) == 8 && plan->dim == 4 && n == 4) return plan->E < 1000;
+    if (sizeof(T) == 8 && plan->dim == 4 && n == 5) return plan->E >= 1000;
+    if (sizeof(T) == 4 && plan->dim == 5 && n == 4) return plan->E < 1000;
+  }
+  return true;
 }
+
+template bool preferred<double>(const gd_plan*, bool, bool);
+template bool preferred<float>(const gd_plan*, bool, bool);
 
 template <typename T>
 int apply(const gd_plan* plan, T mass_coef, T adv_coef, const T* x, T* y, hipStream_t s)

@@ -115,3 +115,14 @@ def test_pinned_where_the_two_node_kernel_also_serves():
     for variant in (KRON, 64):
         op.plan.set_variant(torch.float64, variant)
         assert op.plan.query_variant(torch.float64, 0.0, 1.0) == variant
+
+
+@pytest.mark.parametrize("D,n,dtype,faster", [(4, 4, torch.float64, [5, 5, 5, 5]), (4, 5, torch.float64, [6, 6, 6, 5]),
+                                              (5, 4, torch.float32, [4, 4, 4, 4, 2])], ids=str)
+def test_mass_alone_with_few_points(D, n, dtype, faster):
+    """Mass applies with q = n that the generic kernel does faster keep it: below or above 1,000 elements."""
+    slower = [6, 6, 6, 5] if faster[0] == 5 else [6, 6, 6, 5, 1] if D == 5 else [4] * 4
+    for sizes, sigma, want in ((faster, "poly", KRON), (slower, "poly", 0), (slower, "one", KRON)):
+        fes = G.MakeFiniteElementSpace(G.CartesianMesh(sizes, [1 / s for s in sizes], [0.0] * D, False), G.MakeLobattoFiniteElement(n - 1))
+        op = G.MakeMassFiniteElementOperator(fes, G.MakeIntegrationRule(n), sigma_field("poly", D) if sigma == "poly" else None)
+        assert op.plan.query_variant(dtype, 1.0, 0.0) == want
