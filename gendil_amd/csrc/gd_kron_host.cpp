@@ -357,8 +357,10 @@ bool available(const gd_plan* plan, bool adv, bool mass)
 template <typename T>
 bool preferred(const gd_plan* plan, bool adv, bool mass)
 {
-  // a handful of elements (unit tests, debugging runs) stay on the generic
-  // kernel, which takes the quadrature as it is written
+  // Meshes of up to 64 elements stay on the generic kernel, which callers see as
+  // their variant (tests/test_gpu_n2k.py states it for 2^6 elements); this kernel
+  // would be faster there too (one element, advection, generic against this: 4D
+  // n = 2 16 and 5.8 us, 6D n = 3 76 and 9.2; mass 5.3 and 5.5, 14 and 6).
   if (plan->E <= 64 || !available(plan, adv, mass)) return false;
   // Mass alone with a variable sigma and q = n: the generic kernel interpolates
   // little, and this one holds few elements of these sizes in a CU.  Generic
