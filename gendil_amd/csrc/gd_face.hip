@@ -323,7 +323,7 @@ constexpr int kWaveN = 8;  // largest n and q of either side
 
 __global__ void __launch_bounds__(64) k_interface(Args a)
 {
-  constexpr int W = 64, NN = kWaveN * kWaveN;
+  constexpr int W = 64;
   extern __shared__ double lds[];
   const int q = a.q, qq = q * q, fpb = a.fpb;
   const int64_t f0 = (int64_t)blockIdx.x * fpb;
@@ -334,9 +334,11 @@ __global__ void __launch_bounds__(64) k_interface(Args a)
   const int t0 = a.axis == 0 ? 1 : 0, t1 = a.axis == 2 ? 1 : 2;
   double* B[2] = {lds, lds + q * n[0]};
   double* wq = B[1] + q * n[1];
-  double* X = wq + q;             // [face] traces (nt), then x-tested fluxes (q (n0 + n1))
-  double* Y = X + fpb * 2 * NN;   // [face] y-swept traces (q (n0 + n1)), then the flux is in Z
-  double* Z = Y + fpb * 2 * NN;   // [face] fluxes (q^2)
+  const int rows = n[0] + n[1];
+  const int xp = max(nt, q * rows), yp = q * rows;  // values per face
+  double* X = wq + q;         // [face] traces (nt), then x-tested fluxes (q (n0 + n1))
+  double* Y = X + fpb * xp;   // [face] y-swept traces (q (n0 + n1))
+  double* Z = Y + fpb * yp;   // [face] fluxes (q^2)
   for (int i = lane; i < q * (n[0] + n[1]); i += W) lds[i] = i < q * n[0] ? a.s[0].B[i] : a.s[1].B[i - q * n[0]];
   for (int i = lane; i < q; i += W) wq[i] = a.geo.tab.w[i];
 
@@ -372,18 +374,17 @@ __global__ void __launch_bounds__(64) k_interface(Args a)
     if (sd.node >= 0) v = u[sd.node * sn];
     else
       for (int i = 0; i < m; ++i) v += sd.bf[i] * u[i * sn];
-    X[f * 2 * NN + r] = v;
+    X[f * xp + r] = v;
   }
   __syncthreads();
   // ---- y sweep: [k][i] from [m][i] ----
-  const int rows = n[0] + n[1];
   for (int t = lane; t < nf * q * rows; t += W) {
     const int f = t / (q * rows), r = t - f * (q * rows), k = r / rows, i = r - k * rows;
     const int s = i >= n[0], m = n[s], ii = s ? i - n[0] : i;
-    const double* src = X + f * 2 * NN + (s ? nt0 : 0) + ii;
+    const double* src = X + f * xp + (s ? nt0 : 0) + ii;
     double v = 0.0;
     for (int j = 0; j < m; ++j) v += B[s][k * m + j] * src[j * m];
-    Y[f * 2 * NN + r] = v;
+    Y[f * yp + r] = v;
   }
   __syncthreads();
   // ---- x sweep and the upwind flux at the points of the minus cell ----
@@ -398,21 +399,21 @@ __global__ void __launch_bounds__(64) k_interface(Args a)
     k[t1] = ky;
     k[a.axis] = q + a.xi_minus;
     const double dot = beta_axis(p, a.axis, sub, k, q, 3) * scale;
-    const double* row = Y + f * 2 * NN + ky * rows;
+    const double* row = Y + f * yp + ky * rows;
     double um = 0.0, up = 0.0;
     for (int i = 0; i < n[0]; ++i) um += B[0][kx * n[0] + i] * row[i];
     for (int i = 0; i < n[1]; ++i) up += B[1][kx * n[1] + i] * row[n[0] + i];
-    Z[f * NN + r] = wq[kx] * wq[ky] * p.detJ * (dot > 0.0 ? dot * um : dot * up);
+    Z[f * qq + r] = wq[kx] * wq[ky] * p.detJ * (dot > 0.0 ? dot * um : dot * up);
   }
   __syncthreads();
   // ---- x test ----
   for (int t = lane; t < nf * q * rows; t += W) {
     const int f = t / (q * rows), r = t - f * (q * rows), k = r / rows, i = r - k * rows;
     const int s = i >= n[0], m = n[s], ii = s ? i - n[0] : i;
-    const double* src = Z + f * NN + k * q;
+    const double* src = Z + f * qq + k * q;
     double v = 0.0;
     for (int j = 0; j < q; ++j) v += B[s][j * m + ii] * src[j];
-    X[f * 2 * NN + r] = v;
+    X[f * xp + r] = v;
   }
   __syncthreads();
   // ---- y test, spread along the normal ----
@@ -422,7 +423,7 @@ __global__ void __launch_bounds__(64) k_interface(Args a)
     int s0, s1, sn;
     strides(m, s0, s1, sn);
     const Side& sd = a.s[s];
-    const double* src = X + f * 2 * NN + (s ? n[0] : 0) + i;
+    const double* src = X + f * xp + (s ? n[0] : 0) + i;
     double v = 0.0;
     for (int k = 0; k < q; ++k) v += B[s][k * m + j] * src[k * rows];
     double* yy = sd.y + elem(sd, f) * (m * m * m) + i * s0 + j * s1;
@@ -659,13 +660,14 @@ int launch(const Args& args, hipStream_t st)
   // faces.  (Interior faces by colour and subfaces keep the kernel below, and
   // so do sides that may share elements: this kernel adds both at once, that
   // one after the other.)
-  if (args.D == 3 && args.s[0].stride == 0 && args.s[1].stride == 0 && !args.s[0].Bmap && !args.s[1].Bmap &&
-      args.wscale == 1.0 && std::max({args.s[0].n, args.s[1].n, args.q}) <= kWaveN &&
+  if (args.D == 3 && args.q > 1 && args.s[0].stride == 0 && args.s[1].stride == 0 && !args.s[0].Bmap &&
+      !args.s[1].Bmap && args.wscale == 1.0 && std::max({args.s[0].n, args.s[1].n, args.q}) <= kWaveN &&
       args.nfaces < (1LL << 31) - 64 && !sides_share_elements(args)) {
     Args a = args;
     a.fpb = std::max(1, 64 / (a.q * a.q));
     const long long blocks = (a.nfaces + a.fpb - 1) / a.fpb;
-    const size_t lds = sizeof(double) * (size_t)(a.q * (a.s[0].n + a.s[1].n + 1) + a.fpb * 5 * kWaveN * kWaveN);
+    const int n0 = a.s[0].n, n1 = a.s[1].n, qr = a.q * (n0 + n1);
+    const size_t lds = sizeof(double) * (size_t)(qr + a.q + a.fpb * (std::max(n0 * n0 + n1 * n1, qr) + qr + a.q * a.q));
     if (blocks <= 0x7fffffffLL && lds <= 64 * 1024) {
       hipLaunchKernelGGL(k_interface, dim3((unsigned)blocks), dim3(64), lds, st, a);
       const hipError_t e = hipGetLastError();
