@@ -18,12 +18,13 @@
 // ~47 us), so what is left to save is the time between them.  Each pass leaves
 // one partial per block and column; the next pass sums them in its own prologue,
 // every block for itself in the same fixed order (at most 256 partials of 33
-// columns or 512 of 9: ~64 KB from L2), and pass C's column is finished by one
-// wave of the next step's pass A (or by a one-wave kernel before the cycle's
-// update).  Against one-block finishing kernels between the passes (4-6 us each
-// and a launch gap): the 32^3, p = 3 implicit step in mixed precision (47 cycles of
-// 30) 160.6 -> 145.4 ms.  Walking every second pass downwards for the L2 and
-// loading the first packs before the sums measured the same, with spills.
+// columns, 512 of 9, or 512 of 32 in FP64: 36 to 128 KB from L2), and pass C's
+// column is finished by one wave of the next step's pass A (or by a one-wave
+// kernel before the cycle's update).  Against one-block finishing kernels between
+// the passes (4-6 us each and a launch gap): the 32^3, p = 3 implicit step in
+// mixed precision (47 cycles of 30) 160.6 -> 145.4 ms.  Walking every second pass
+// downwards for the L2 and loading the first packs before the sums measured the
+// same, with spills.
 //
 // The residual estimate |g_{k+1}| goes to the caller's pointer (pinned host
 // memory, so a host loop can poll it with no copy or event in the stream) from
@@ -33,9 +34,11 @@
 //
 // Bases are read 16 bytes per lane where the basis and its leading dimension
 // are 16-byte aligned (pass B in FP32, which keeps every loaded value live, 8
-// bytes): one block per CU needs that many bytes in flight (FP64 32^3, p = 3 with
-// 8 bytes per lane 315 ms a solve, with 16 300; 296 with the finishing kernels,
-// which smaller systems beat: 16^3 81.3 -> 64.1, 28^3 p = 2 42.8 -> 37.5).
+// bytes): one block per CU needs that many bytes in flight (with 8 in FP64 a solve
+// took 5 % longer).  FP64 passes A and C take two blocks per CU for any number of
+// vectors (pass B's registers hold one): FP64 solves, 32^3, p = 3 (1885 iterations)
+// 402 ms with one block, 376 with two (399 with the finishing kernels), 16^3 81,
+// 80 (103), 28^3, p = 2 41.9, 40.6 (47.3).
 //
 // The cycle end solves the triangular system H y = g in one wave (with the last
 // column's finish) and adds x += sum_j s_j y_j V_j in FP64.
@@ -57,6 +60,9 @@ constexpr int kMaxBlocks = 512;     // partials per column
 // blocks of a pass over KK vectors: two per CU while there are few loads per
 // thread (and few columns to sum), else one
 constexpr int max_blocks(int KK) { return KK <= 8 ? kMaxBlocks : kMaxBlocks / 2; }
+// of passes A and C: more in flight for FP64 vectors, twice as long
+template <typename TV>
+constexpr int max_blocks_ac(int KK) { return sizeof(TV) == 8 ? kMaxBlocks : max_blocks(KK); }
 
 struct Workspace {
   double H[kMaxM][kMaxM + 1];  // column k, rows 0..k+1 (rotated)
@@ -125,30 +131,34 @@ __device__ __forceinline__ void store_block_partials(const double (&acc)[K], dou
 }
 
 // col[j] = sum over nblk <= MAXB partials of column j, j < K: TPC threads per
-// column, all their loads in flight together, then a shuffle sum; a fixed order
-// for a given grid.  Visible to every thread on return.
+// column, the loads of 256 partials in flight together, then a shuffle sum; a
+// fixed order for a given grid.  Visible to every thread on return.
 template <int K, int MAXB>
 __device__ __forceinline__ void sum_columns(const double (*partial)[kMaxBlocks], int nblk, double* col)
 {
   constexpr int TPC = K <= 8 ? 64 : K <= 16 ? 32 : 16;
   constexpr int CPP = kThreads / TPC;  // columns per round
-  constexpr int PER = MAXB / TPC;      // partials per thread
+  constexpr int ROUND = MAXB < 256 ? MAXB : 256;
+  constexpr int PER = ROUND / TPC;     // partials per thread and round
   const int lane = threadIdx.x % TPC, c0 = threadIdx.x / TPC;
 #pragma unroll
   for (int r = 0; r < (K + CPP - 1) / CPP; ++r) {
     const int j = c0 + r * CPP;
     if (j < K) {  // uniform over each group of TPC threads; the shuffles stay inside it
       const double* cp = partial[j];
-      double v[PER];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int bb = lane + TPC * i;
-        const double x = cp[bb < nblk ? bb : nblk - 1];
-        v[i] = bb < nblk ? x : 0.0;
-      }
       double sum = 0.0;
+#pragma unroll 1
+      for (int b0 = 0; b0 < nblk; b0 += ROUND) {  // nblk is the same in every thread
+        double v[PER];
 #pragma unroll
-      for (int i = 0; i < PER; ++i) sum += v[i];
+        for (int i = 0; i < PER; ++i) {
+          const int bb = b0 + lane + TPC * i;
+          const double x = cp[bb < nblk ? bb : nblk - 1];
+          v[i] = bb < nblk ? x : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) sum += v[i];
+      }
 #pragma unroll
       for (int off = TPC / 2; off > 0; off >>= 1) sum += __shfl_down(sum, off, TPC);
       if (lane == 0) col[j] = sum;
@@ -243,12 +253,12 @@ __global__ void __launch_bounds__(kThreads) k_pass_a(int64_t n, const TV* __rest
 
 // Pass B: h1_j = s_j <V_j, W>, c_j = s_j h1_j; W -= sum_j c_j V_j; partial row = <V_j, W_new>, ||W_new||^2.
 template <typename TV, int KK, int W>
-__global__ void __launch_bounds__(kThreads) k_pass_b(int64_t n, TV* __restrict__ V, int64_t ldv,
+__global__ void __launch_bounds__(kThreads) k_pass_b(int64_t n, TV* __restrict__ V, int64_t ldv, int na,
                                                      Workspace* __restrict__ ws)
 {
   TV* __restrict__ w = V + (int64_t)KK * ldv;
   __shared__ double col[KK];
-  sum_columns<KK, max_blocks(KK)>(ws->pa, gridDim.x, col);
+  sum_columns<KK, max_blocks_ac<TV>(KK)>(ws->pa, na, col);
   double c_l = 0.0;
   {
     const int j = threadIdx.x & 63;
@@ -312,12 +322,12 @@ __global__ void __launch_bounds__(kThreads) k_pass_b(int64_t n, TV* __restrict__
 // p = sqrt(||W||^2 - sum_j h2_j^2); Z = (W - sum_j c_j V_j) / p stored as V_KK;
 // partial = ||Z||^2.
 template <typename TV, int KK, int W>
-__global__ void __launch_bounds__(kThreads) k_pass_c(int64_t n, TV* __restrict__ V, int64_t ldv,
+__global__ void __launch_bounds__(kThreads) k_pass_c(int64_t n, TV* __restrict__ V, int64_t ldv, int nb,
                                                      Workspace* __restrict__ ws, double* resid_out)
 {
   TV* __restrict__ w = V + (int64_t)KK * ldv;
   __shared__ double col[KK + 1];
-  sum_columns<KK + 1, max_blocks(KK)>(ws->pb, gridDim.x, col);
+  sum_columns<KK + 1, max_blocks(KK)>(ws->pb, nb, col);
   double c_l = 0.0, h2 = 0.0;
   const int lane = threadIdx.x & 63;
   if (lane < KK) {
@@ -478,10 +488,10 @@ int step(int64_t n, int m, int k, TV* V, int64_t ldv, void* wsp, double* resid_o
     constexpr int WB = W < 2 ? W : 2;
     with_count<1>(k + 1, [&](auto KK_) {
       constexpr int KK = decltype(KK_)::value;
-      const int nb = grid_for(n, W, max_blocks(KK));
-      hipLaunchKernelGGL((k_pass_a<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws);
-      hipLaunchKernelGGL((k_pass_b<TV, KK, WB>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws);
-      hipLaunchKernelGGL((k_pass_c<TV, KK, W>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, ws, resid_out);
+      const int nb = grid_for(n, W, max_blocks(KK)), na = grid_for(n, W, max_blocks_ac<TV>(KK));
+      hipLaunchKernelGGL((k_pass_a<TV, KK, W>), dim3(na), dim3(kThreads), 0, st, n, V, ldv, ws);
+      hipLaunchKernelGGL((k_pass_b<TV, KK, WB>), dim3(nb), dim3(kThreads), 0, st, n, V, ldv, na, ws);
+      hipLaunchKernelGGL((k_pass_c<TV, KK, W>), dim3(na), dim3(kThreads), 0, st, n, V, ldv, nb, ws, resid_out);
     });
   };
   if (packed<TV>(V, ldv)) launch(std::integral_constant<int, kPack<TV>>{});
