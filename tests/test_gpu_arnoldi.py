@@ -15,17 +15,28 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,m,stop", [(700, 32, 32), (70_003, 32, 32), (70_003, 32, 9), (4_300_007, 32, 32),
                                       (4_300_007, 9, 8), (70_003, 5, 1)])
 def test_cycle_minimises_the_residual(n, m, stop, dtype):
+    check_cycle(n, m, stop, dtype, n + (-n) % 4, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,m,stop", [(700, 32, 32), (70_003, 32, 9), (70_003, 5, 1), (4_300_007, 32, 32)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_cycle_on_a_basis_that_no_16_bytes_align(n, m, stop, dtype, offset):
+    """One value per access: an odd leading dimension, and V and x one element off."""
+    check_cycle(n, m, stop, dtype, n + 1 - n % 2, offset)
+
+
+def check_cycle(n, m, stop, dtype, ldv, offset):
     lib = L.lib()
     st = torch.cuda.current_stream().cuda_stream
     g = torch.Generator(device="cuda").manual_seed(n + m)
     d = 1.0 + torch.rand(n, generator=g, device="cuda", dtype=torch.float64)
     b = torch.randn(n, generator=g, device="cuda", dtype=torch.float64)
-    ldv = n + (-n) % 4
-    V = torch.zeros((m + 1, ldv), dtype=dtype, device="cuda")
+    V = torch.zeros(offset + (m + 1) * ldv, dtype=dtype, device="cuda")[offset:].view(m + 1, ldv)
     ws = torch.randint(0, 255, (lib.gd_gmres_workspace_bytes(),), generator=g, dtype=torch.uint8, device="cuda")
     step = lib.gd_arnoldi_step_f64 if dtype == torch.float64 else lib.gd_arnoldi_step_f32
     upd = lib.gd_gmres_update_f64 if dtype == torch.float64 else lib.gd_gmres_update_f32
-    x = torch.zeros(n, dtype=torch.float64, device="cuda")
+    x = torch.zeros(offset + n, dtype=torch.float64, device="cuda")[offset:]
     # the check's own sums of n products round like a walk of n steps, sqrt(n) eps
     # (4.6e-13 at the largest n: the first vector, normalised by torch, shows 6e-14)
     tol = max(1e-13, n**0.5 * 2.0**-52) if dtype == torch.float64 else 1e-6
