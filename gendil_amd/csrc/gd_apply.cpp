@@ -70,7 +70,7 @@ int check_adv(const gd_plan* plan, bool need_pointwise)
 // else the staged Kronecker kernel, else the register Kronecker kernel, else
 // the register kernel, else (apply_impl) the plane kernel, code 72, for any
 // other basis, rule and separable or affine field it is compiled for: 2 to 5
-// times the generic kernel's speed (53 x 47 x 41, p = 3, q = 5: 92 against 438 us).
+// times the generic kernel's speed (53 x 47 x 41, p = 3, q = 5: 90 against 438 us).
 template <typename T>
 int k3_choice(const gd_plan* plan, int N, bool adv, bool mass)
 {

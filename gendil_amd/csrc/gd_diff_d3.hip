@@ -1,8 +1,8 @@
 // SIPDG diffusion kernel instances for 3D meshes: (nodes, points) of GenDiL's
 // diffusion tests (GLL, q = p + 3: test-diffusion-3d-generic.cpp:78-100), of
 // q = p + 2 (examples/poisson) and of q = p + 1.  The plane kernel (gd_dplane.hpp)
-// takes these first; what it leaves here are small FP64 meshes with q >= 4 and
-// meshes of 2^31 elements and more.
+// takes these first; what it leaves here are small FP64 meshes with q >= 4,
+// meshes of 2^31 elements and more, and plans on which variant 0 is pinned.
 #include "gd_diff.hpp"
 
 namespace gd {

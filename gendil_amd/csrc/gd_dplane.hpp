@@ -16,7 +16,7 @@
 // (z-contracted, n values each); of a z face: J, S.  The outputs overwrite the
 // first two fields.
 //
-// 64^3, p = 3, q = 5, an eight-term diffusivity, FP64: 447 us against 940 us for
+// 64^3, p = 3, q = 5, an eight-term diffusivity, FP64: 441 us against 940 us for
 // the generic diffusion kernel (every contraction through LDS); 27 x 23 x 19,
 // p = 2, q = 4, FP32: 9.4 against 25.9 us.  Bound by waits at six waves a CU
 // (4 KB of LDS per element; 197 us of VALU issue): with two cell waves a block

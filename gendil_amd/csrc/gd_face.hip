@@ -315,9 +315,8 @@ __global__ void __launch_bounds__(kThreads) k_faces(Args a)
 // fluxes as k_faces; a face set is small (one layer of cells), so the kernel is
 // bound by its chain of phases, not by throughput: both sides go through each
 // phase together (load, y sweep, x sweep and flux, x test, y test and add: four
-// LDS exchanges inside one wave instead of fourteen block barriers), the old
-// values of y and the field are read at the start, and a launch has a wave per
-// floor(64 / q^2) faces.  40 x 36 x 32, p = 1 | p = 3, 5 points (1,152 faces):
+// LDS exchanges inside one wave instead of fourteen block barriers), and a launch
+// has a wave per floor(64 / q^2) faces.  40 x 36 x 32, p = 1 | p = 3, 5 points (1,152 faces):
 // 17.8 -> 8.9 us.
 constexpr int kWaveN = 8;  // largest n and q of either side
 

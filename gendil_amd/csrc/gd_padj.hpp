@@ -184,19 +184,32 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
   }
   __syncthreads();
 
-  // the field on a face as its flux takes it: outflow only at the boundary (none
-  // at all without data), where nothing else enters
-  auto face_beta = [&](double beta, bool upper, bool bnd) {
-    const double out = a.bc_none ? 0.0 : (upper ? fmax(beta, 0.0) : fmin(beta, 0.0));
-    return bnd ? out : beta;
+  // Which values of dot = beta . n give a face its flux: on an inner face all but
+  // the negative (what is not a number stays so), at the boundary the positive
+  // only, without data none.  Kept as the face's floating-point classes (the sign
+  // bit marks the boundary) or as a flag, whichever leaves the registers better
+  // off.  Transpose with the classes and with the flag, us: 80^3, n = 2, q = 3 137
+  // and 141; 64^3, n = 3, q = 5 353 and 336; 56^3, n = 4, q = 6 362 and 380; 48^3, n =
+  // 5, q = 5 218 and 217 (with the rule where the field is read 258: its loads are
+  // waited for there).  Conditions that branch around the flux gain up to 16 % on
+  // large meshes of n < 5, but cost 8 to 16 % on 12^3 elements and a third at n = 5.
+  auto face_rule = [&](int nb) {
+    constexpr int nan = 0x3, zero = 0x60, positive = 0x380;
+    if constexpr (N % 2 == 0) return nb >= 0 ? nan | zero | positive : (a.bc_none ? 0 : positive) | (1 << 31);
+    else return nb < 0;
   };
-  // the flux of one face point that this side's test function collects:
-  // outflow c dot (own - nb), as the neighbour tests its inflow with -dot
-  // (unless dot < 0: what is not a number stays so)
-  auto flux = [&](double c, double beta, bool upper, bool bnd, double own, double nb) {
+  // the flux of one face point that this side's test function collects: outflow
+  // c dot (own - nb), as the neighbour tests its inflow with -dot
+  auto flux = [&](double c, double beta, bool upper, auto rule, double own, double nb) {
     const double dot = upper ? beta : -beta;
-    const double v = bnd ? own : own - nb;
-    return dot < 0.0 ? 0.0 : c * dot * v;
+    if constexpr (N % 2 == 0) {
+      const double v = rule < 0 ? own : own - nb;
+      return __builtin_amdgcn_class(dot, rule) ? c * dot * v : 0.0;
+    } else {
+      const double v = own - nb;  // nb is 0 at the boundary
+      const bool skip = (rule && a.bc_none) | (rule & (dot != dot));
+      return !(dot <= 0.0) & !skip ? c * dot * v : 0.0;
+    }
   };
 
   // ---- phase 2 ----
@@ -219,17 +232,17 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
         }
       double xn[2][Q];  // the x neighbours' traces at the rows
       double fx[2][Q];  // beta on the x faces
-      bool xb[2];
+      decltype(face_rule(0)) xr[2];
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const double* src = a.beta_face[0] + face_index(a, sub, 0, s) * QQ + kz * Q;
-        xb[s] = mesh.neighbour(e, sub, 0, s) < 0;
 #pragma unroll
-        for (int k = 0; k < Q; ++k) fx[s][k] = face_beta(src[k], s, xb[s]);
+        for (int k = 0; k < Q; ++k) fx[s][k] = src[k];
         double nd[N];
 #pragma unroll
         for (int m = 0; m < N; ++m) nd[m] = r[2 * NN + s * N + m];
         P::up(B, nd, xn[s]);
+        xr[s] = face_rule(mesh.neighbour(e, sub, 0, s));
       }
 #pragma unroll
       for (int k = 0; k < Q; ++k) {
@@ -257,8 +270,8 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
         for (int j = 0; j < Q; ++j) f[j] = (f[j] - a.c[2] * bz[j] * g[j]) * (wz * w[k] * w[j]);
         P::down(B, f, o);
         const double cw = a.c[0] * wz * w[k];
-        const double lo = flux(cw, fx[0][k], false, xb[0], end_of<N, GLL>(t0, 0, b0, b1), xn[0][k]);
-        const double hi = flux(cw, fx[1][k], true, xb[1], end_of<N, GLL>(t0, 1, b0, b1), xn[1][k]);
+        const double lo = flux(cw, fx[0][k], false, xr[0], end_of<N, GLL>(t0, 0, b0, b1), xn[0][k]);
+        const double hi = flux(cw, fx[1][k], true, xr[1], end_of<N, GLL>(t0, 1, b0, b1), xn[1][k]);
         if constexpr (GLL) {
           o[0] += lo;
           o[N - 1] += hi;
@@ -274,10 +287,9 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
       for (int s = 0; s < 2; ++s) {  // y faces
         const double* src = a.beta_face[1] + face_index(a, sub, 1, s) * QQ + kz * Q;
-        const bool bnd = mesh.neighbour(e, sub, 1, s) < 0;
         double be[Q], nd[N], own[Q], ext[Q], f[Q], o[N];
 #pragma unroll
-        for (int k = 0; k < Q; ++k) be[k] = face_beta(src[k], s, bnd);
+        for (int k = 0; k < Q; ++k) be[k] = src[k];
         pin(A);
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -292,8 +304,9 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
 #pragma unroll
         for (int i = 0; i < N; ++i) nd[i] = r[2 * NN + (2 + s) * N + i];
         P::up(B, nd, ext);
+        const auto rule = face_rule(mesh.neighbour(e, sub, 1, s));
 #pragma unroll
-        for (int j = 0; j < Q; ++j) f[j] = flux(a.c[1] * wz * w[j], be[j], s, bnd, own[j], ext[j]);
+        for (int j = 0; j < Q; ++j) f[j] = flux(a.c[1] * wz * w[j], be[j], s, rule, own[j], ext[j]);
         P::down(B, f, o);
         if constexpr (GLL) {
 #pragma unroll
@@ -338,27 +351,28 @@ __global__ void __launch_bounds__((AdjGeo<N, Q>::NT)) __attribute__((amdgpu_wave
       mesh.decode(e, sub);
       double* r = zrec + (el * 2 + s) * ZP;
       const double* src = a.beta_face[2] + face_index(a, sub, 2, s) * QQ;
-      const bool bnd = mesh.neighbour(e, sub, 2, s) < 0;
+      const int nb = mesh.neighbour(e, sub, 2, s);
+      const auto rule = face_rule(nb);
       double u[N][N], A[N][N];
       // the flux takes own - nb, one interpolation of the difference
 #pragma unroll
       for (int m = 0; m < N; ++m)
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          u[m][i] = bnd ? r[m * N + i] : r[m * N + i] - r[NN + m * N + i];
+          u[m][i] = nb < 0 ? r[m * N + i] : r[m * N + i] - r[NN + m * N + i];
           A[m][i] = 0.0;
         }
 #pragma unroll
       for (int k = 0; k < Q; ++k) {
         double be[Q], t0[N], f[Q], o[N];
 #pragma unroll
-        for (int j = 0; j < Q; ++j) be[j] = face_beta(src[k * Q + j], s, bnd);
+        for (int j = 0; j < Q; ++j) be[j] = src[k * Q + j];
         pin(A);
         pin(u);
         P::row(B, u, k, t0);
         P::up(B, t0, f);
 #pragma unroll
-        for (int j = 0; j < Q; ++j) f[j] = flux(a.c[2] * (w[k] * w[j]), be[j], s, bnd, f[j], 0.0);
+        for (int j = 0; j < Q; ++j) f[j] = flux(a.c[2] * (w[k] * w[j]), be[j], s, rule, f[j], 0.0);
         P::down(B, f, o);
 #pragma unroll
         for (int m = 0; m < N; ++m)

@@ -248,6 +248,24 @@ def test_nan_in_a_pointwise_face_field_reaches_the_transpose():
         assert np.array_equal(np.isnan(got), np.isnan(want))
 
 
+@pytest.mark.parametrize("n,q", PAIRS)
+def test_nan_in_a_pointwise_boundary_field_gives_no_outflow(n, q):
+    """NaN at a point of one boundary face per axis, with data: the transpose takes it as no outflow."""
+    fes, ir = space((5, 3, 4), n - 1, "G", False), G.MakeIntegrationRule(q)
+    cell, faces, _ = pointwise_problem(fes, q, 4)
+    for a, f in enumerate((5, 3 * 5, 4 * 15)):  # an upper boundary face
+        faces[a][f, 1] = np.nan
+    dev = [torch.as_tensor(t, device="cuda") for t in (cell, *faces)]
+    op = G.MakeAdvectionOperator(fes, ir, G.PointwiseField(dev[0], dev[1:]), bc_field("poly", 3))
+    r = G.fill_random(op.num_dofs, 22)
+    dr = torch.as_tensor(r, device="cuda")
+    got = op.transpose(dr, torch.empty_like(dr)).cpu().numpy()
+    for f in faces:
+        f[np.isnan(f)] = 0.0
+    want = oracle.Problem(fes, ir, adv_coef=1.0, adv=(cell, faces), bc=bc_field("poly", 3)).apply_transpose(r)
+    assert rel_l2(got, want) <= 1e-12
+
+
 def pinned(op, dtype, run):
     """run() by default and with the generic kernel pinned: other sums, so other last bits."""
     default = run()
